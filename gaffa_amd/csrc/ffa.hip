@@ -12,10 +12,12 @@
 //             workgroup stages a contiguous input span in LDS with coalesced
 //             loads, then each output is summed serially in the CPU's FP32
 //             order
-//   subtree   persistent, one workgroup per CU walking (node at the task's
-//             LDS depth D, series) units: the node's rows live in LDS and
-//             every level below it runs there, ping-ponging between two LDS
-//             buffers, with merges from host-built tables
+//   subtree   persistent workgroups walking (node at the task's LDS depth D,
+//             series) units.  Plans of up to 304 bins: two workgroups per CU,
+//             each wave runs one of the node's eight sub-nodes in registers
+//             and the top three levels merge from LDS.  Other plans: one
+//             workgroup per CU, every level in LDS between two buffers, with
+//             merges from host-built tables
 //   level     one launch per output depth: one to three levels per pass,
 //             each item (32 rows of one node) copying its leaf rows' runs
 //             from HBM into LDS and merging there
@@ -26,8 +28,8 @@
 //             P[phi + w], so every boxcar sum equals the CPU's circular-prefix
 //             difference bit for bit (ffa_detection.cpp:126-239); significant
 //             peaks are appended with one atomic each.
-// The subtree and level kernels read their merges and leaves from host-built
-// tables; in the terminal kernel the (head row, tail row, roll) descriptor of
+// The LDS subtree and level kernels read their merges and leaves from
+// host-built tables; in the terminal kernel the (head row, tail row, roll) descriptor of
 // each output row is computed once, by one lane, into LDS.  The waves then
 // stream whole rows (lanes over phase bins) reading only those.  The subtree
 // and level passes write their rows with streaming stores.
@@ -54,8 +56,8 @@ constexpr uint32_t kMaxLdsBytes = 160 * 1024;
 
 // ffa.cpp:133-143 in FP32, no contraction (the library is built with
 // -ffp-contract=off).
-__host__ __device__ __forceinline__ uint32_t pick_row(uint32_t child_rows, uint32_t rows,
-                                             uint32_t s) {
+__host__ __device__ __forceinline__ constexpr uint32_t pick_row(uint32_t child_rows, uint32_t rows,
+                                                       uint32_t s) {
   const float scale = static_cast<float>(child_rows - 1) / static_cast<float>(rows - 1);
   return static_cast<uint32_t>(scale * static_cast<float>(s) + 0.5f);
 }
@@ -340,8 +342,9 @@ ffa_prepare_fused_kernel(const float* __restrict__ series, uint64_t series_strid
 }
 
 // ------------------------------------------------------------- subtree ----
-// Persistent: one workgroup per CU walks the (node, series) units of the
-// launch, unit u = (subtree item u % nitems, series u / nitems), so that the
+// Plans with nodes of more than kNodeMaxRows rows (few bins) or more than
+// kNodeMaxBins bins.  Persistent: one workgroup per CU walks the (node, series)
+// units of the launch, unit u = (subtree item u % nitems, series u / nitems), so that the
 // units in flight together share a series' prepared data in L2.  For each
 // unit: the node's rows, prefetched into registers while the previous unit
 // computed, are written to LDS; the levels run in LDS (ping-pong), the top
@@ -604,6 +607,420 @@ ffa_subtree_kernel(KArgs a, uint32_t nunits) {
       else level(One{}, table, cur, to_global);
     }
     __syncthreads();  // the LDS rows are rewritten by the next unit
+  }
+}
+
+// -------------------------------------------------- subtree, registers ----
+// The subtree kernel of plans whose nodes all hold at most kNodeMaxRows rows of
+// at most kNodeMaxBins bins: beyond them a sub-node no longer fits 64 registers
+// per lane (rows x C), and ffa_subtree_kernel runs the plan.  A 512-thread workgroup runs one (node, series) unit
+// at a time, two workgroups per CU:
+//   1. wave w owns the node's depth-3 sub-node w (ceil(rows / 8) rows at most)
+//      and runs all of its levels in registers.  Lane l holds phases l C ..
+//      l C + C - 1 of every row (the phases past the row's end being its
+//      circular extension), so a roll r is a
+//      renaming of registers plus (c + r) / C one-lane shifts (DPP), and the
+//      sub-node's tree is known at compile time: one add per value and level,
+//      no LDS access and no address arithmetic;
+//   2. the sub-node's rows go to LDS (one buffer) and after a barrier each wave
+//      merges the node's top three levels from eight LDS rows per output row,
+//      straight into the work region.  A roll of row s is at most s, so only
+//      the row's last one or two 64-phase chunks can wrap and need a choice of
+//      address.  Output rows go in pairs (2 i, 2 i + 1): in an even node both
+//      read the same head and tail rows one phase apart, in an odd one they
+//      share one of the two, so 8 or 12 LDS rows serve two output rows.
+// Two barriers per unit instead of one per two tree levels, and the node takes
+// half the LDS, so that one workgroup's loads and barriers hide behind the
+// other's work.  The tree in registers costs nothing measurable (a build
+// without it took the same time); what bounds the kernel is the loads and LDS
+// stores of step 1 (about half its time) and VALU issue in step 2 (60 % busy).
+// Measured against ffa_subtree_kernel, which it replaces here: 64 series of
+// 2^21 samples (bins 180..256, per launch) 11.5 -> 6.0 ms, 256 series of 2^20
+// 24.8 -> 13.8 ms, 96 octave-plan series of 2^18..2^20 (bins 128..255) 5.4 ->
+// 2.7 ms.  Steps on the way at the middle shape: dword loads 17.6 ms, one load
+// per lane and row 15.1, row pairs 14.1, integer row selection 13.7.
+constexpr uint32_t kNodeThreads = 512;
+constexpr uint32_t kNodeWaves = kNodeThreads / 64;  // sub-nodes of a node (depth 3)
+constexpr uint32_t kNodeMaxRows = 160;
+constexpr uint32_t kNodeMinBins = 64;
+constexpr uint32_t kNodeMaxBins = 304;
+constexpr uint32_t kNodeRegs = 64;   // floats of a sub-node per lane: rows x C
+constexpr uint32_t kNodeGuard = 64;  // floats of LDS slack: the last chunk of a row overreads
+constexpr uint32_t kNodeMaxSub = (kNodeMaxRows + kNodeWaves - 1) / kNodeWaves;
+constexpr uint32_t kNodeMaxC = 5;
+
+// Largest sub-node of C registers per row and lane.
+constexpr uint32_t node_max_sub(uint32_t c) {
+  return kNodeRegs / c < kNodeMaxSub ? kNodeRegs / c : kNodeMaxSub;
+}
+
+// Registers per row and lane for a node of `rows` rows of `bins` bins; 0 where
+// the unit takes the generic path (too few rows for eight sub-nodes, or a row
+// shorter than its sub-node's rolls).
+__host__ __device__ __forceinline__ uint32_t node_regs_per_row(uint32_t rows, uint32_t bins) {
+  if (rows < kNodeWaves || rows > kNodeMaxRows || bins < kNodeMinBins || bins > kNodeMaxBins)
+    return 0;
+  const uint32_t sub = (rows + kNodeWaves - 1) / kNodeWaves;
+  uint32_t c = 2;
+  // up to c - 1 phases in front of the row, then the row and its extension
+  while (64 * c < bins + sub - 1 + (c - bins % c) % c) ++c;
+  return c > kNodeMaxC || sub > node_max_sub(c) ? 0 : c;
+}
+
+// Dynamic LDS of a launch whose largest node holds `half` floats: one row
+// buffer, or two of the small nodes that take the generic path.
+__host__ __forceinline__ uint32_t node_lds_bytes(uint32_t half) {
+  return 4u * std::max(half + kNodeGuard, std::min(2u * half, 2u * kNodeMaxRows * kNodeMinBins));
+}
+
+// pick_row(child, n, s) for the children of a node of n <= kNodeMaxRows rows, in
+// integers: both children of an even node and the tail of an odd one take s / 2
+// rounded down and up, and the head of an odd one s / 2 rounded down, less one for
+// even s past the middle.
+constexpr uint32_t below_row(uint32_t n, bool tail, uint32_t s) {
+  const uint32_t odd = n & 1u;
+  return tail ? (s + odd) >> 1 : (s - (odd != 0 && s > n / 2 ? 1u : 0u)) >> 1;
+}
+constexpr bool below_row_is_pick_row(uint32_t lo, uint32_t hi) {
+  for (uint32_t n = lo; n < hi; ++n)
+    for (uint32_t s = 0; s < n; ++s)
+      if (below_row(n, false, s) != pick_row(n / 2, n, s) ||
+          below_row(n, true, s) != pick_row(n - n / 2, n, s))
+        return false;
+  return true;
+}
+static_assert(below_row_is_pick_row(2, 100) && below_row_is_pick_row(100, 140) &&
+                  below_row_is_pick_row(140, kNodeMaxRows + 1),
+              "the integer row selection is the FP32 one");
+
+// x of the next lane (lane 63 gets 0).
+__device__ __forceinline__ float next_lane(float x) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x130 /* wave_shl:1 */,
+                                         0xf, 0xf, true));
+}
+
+// A row in 64-phase chunks, one phase further: x of the next lane, and in lane
+// 63 lane 0 of the next chunk.
+__device__ __forceinline__ float next_phase(float x, float next_chunk) {
+  const int wrapped = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, next_chunk),
+                                                  0x134 /* wave_rol:1 */, 0xf, 0xf, false);
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(wrapped, __builtin_bit_cast(int, x), 0x130, 0xf, 0xf,
+                                         false));
+}
+
+// The tree of N rows starting at row S of v (C registers per row), in place.
+template <uint32_t C, uint32_t S, uint32_t N, uint32_t SIZE>
+__device__ __forceinline__ void register_tree(float (&v)[SIZE]) {
+  if constexpr (N > 1) {
+    constexpr uint32_t H = N / 2, T = N - H;
+    register_tree<C, S, H>(v);
+    register_tree<C, S + H, T>(v);
+    float out[N * C];
+#pragma unroll
+    for (uint32_t s = 0; s < N; ++s) {
+      const uint32_t h = pick_row(H, N, s), t = pick_row(T, N, s), roll = s - t;
+#pragma unroll
+      for (uint32_t c = 0; c < C; ++c) {
+        float x = v[(S + H + t) * C + (c + roll) % C];
+#pragma unroll
+        for (uint32_t k = 0; k < (c + roll) / C; ++k) x = next_lane(x);
+        out[s * C + c] = v[(S + h) * C + c] + x;
+      }
+      // row order: an input row dies as soon as its last output row is done
+      if constexpr (N * C > 24) __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (uint32_t e = 0; e < N * C; ++e) v[S * C + e] = out[e];
+    if constexpr (N * C > 8) __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// Loads the wave's `n` rows of `b` phases, runs their tree and, once every wave
+// is done with the previous unit's LDS rows, writes them to dst[0 .. n).  p0 is
+// the lane's first phase: lane C - o, with o < C such that the row's end falls
+// between two lanes (so a lane's C phases are one load); lane 0's o phases in
+// front of the row hold another row's end, and nothing reads them.
+template <uint32_t C, uint32_t N = 1>
+__device__ __forceinline__ void run_sub_node(uint32_t n, const float* row, float* dst, uint32_t b,
+                                             int32_t p0, bool first_row) {
+  if (n == N) {
+    float v[N * C];
+    // ext_vector_type(3) is padded to 16 bytes: three floats as a struct
+    struct Lane {
+      float x[C];
+    };
+    const uint32_t at = static_cast<uint32_t>(p0 < static_cast<int32_t>(b) ? p0 : p0 - b);
+#pragma unroll
+    for (uint32_t r = 0; r < N; ++r) {
+      if (r == 0 && first_row) {
+        // the input's first row: lane 0 must not read in front of it
+#pragma unroll
+        for (uint32_t c = 0; c < C; ++c) v[c] = row[max(static_cast<int32_t>(at + c), 0)];
+      } else {
+        const Lane q = *reinterpret_cast<const Lane*>(row + static_cast<int32_t>(at));
+#pragma unroll
+        for (uint32_t c = 0; c < C; ++c) v[r * C + c] = q.x[c];
+      }
+      row += b;
+    }
+    register_tree<C, 0, N>(v);
+    // the adds stay here: moved into the conditional stores below, they would
+    // keep their operands' registers alive
+#pragma unroll
+    for (uint32_t e = 0; e < N * C; ++e) asm volatile("" : "+v"(v[e]));
+    __syncthreads();
+#pragma unroll
+    for (uint32_t c = 0; c < C; ++c) {
+      const uint32_t p = static_cast<uint32_t>(p0) + c;
+      if (p < b) {
+        float* d = dst + p;
+#pragma unroll
+        for (uint32_t r = 0; r < N; ++r, d += b) *d = v[r * C + c];
+      }
+    }
+  } else if constexpr (N < node_max_sub(C)) {
+    run_sub_node<C, N + 1>(n, row, dst, b, p0, first_row);
+  }
+}
+
+// f(integral_constant<C>) for the run-time register count c in 2 .. kNodeMaxC.
+template <typename F>
+__device__ __forceinline__ void with_regs_per_row(uint32_t c, F&& f) {
+  static_assert(kNodeMaxC == 5, "one case per register count");
+  if (c == 4) f(std::integral_constant<uint32_t, 4>{});
+  else if (c == 3) f(std::integral_constant<uint32_t, 3>{});
+  else if (c == 5) f(std::integral_constant<uint32_t, 5>{});
+  else f(std::integral_constant<uint32_t, 2>{});
+}
+
+__global__ void __launch_bounds__(kNodeThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
+ffa_node_kernel(KArgs a, uint32_t nunits) {
+  extern __shared__ float lds[];
+  const gaffa_hip_ffa_plan_desc& plan = a.plan;
+  const uint32_t tid = threadIdx.x;
+  const uint32_t lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t nitems = plan.nsubtree_items;
+  using ConstItem = __attribute__((address_space(4))) const gaffa_hip_ffa_item;
+  using ConstTask = __attribute__((address_space(4))) const gaffa_hip_ffa_task;
+  using ConstGroup = __attribute__((address_space(4))) const gaffa_hip_ffa_group;
+  ConstItem* const items = (ConstItem*)plan.subtree_items;
+  ConstTask* const tasks = (ConstTask*)plan.tasks;
+  ConstGroup* const groups = (ConstGroup*)plan.groups;
+
+  auto input_rows = [&](ConstItem* it, ConstTask* t, uint64_t series) {
+    ConstGroup* g = groups + t->group;
+    return (g->factor == 1.0 ? a.series + series * a.series_stride + g->input_offset
+                             : a.prepared + series * plan.prepared_stride + g->prep_offset) +
+           static_cast<uint64_t>(it->a) * t->bins;
+  };
+  // the wave's depth-3 sub-node of a node of `rows` rows: first row and rows
+  auto sub_node = [&](uint32_t rows, uint32_t& first) {
+    first = 0;
+#pragma unroll
+    for (int32_t k = 2; k >= 0; --k) {
+      const uint32_t h = rows / 2;
+      const bool tail = (wave >> k) & 1u;
+      first += tail ? h : 0u;
+      rows = tail ? rows - h : h;
+    }
+    return rows;
+  };
+
+  // unit u = item + nitems * series, stepped without divisions in the loop
+  const uint32_t item_step = __builtin_amdgcn_readfirstlane(gridDim.x % nitems);
+  const uint32_t series_step = __builtin_amdgcn_readfirstlane(gridDim.x / nitems);
+  uint32_t item = __builtin_amdgcn_readfirstlane(blockIdx.x % nitems);
+  uint64_t sidx = __builtin_amdgcn_readfirstlane(blockIdx.x / nitems);
+  for (uint32_t u = blockIdx.x; u < nunits; u += gridDim.x, item += item_step, sidx += series_step) {
+    if (item >= nitems) {
+      item -= nitems;
+      ++sidx;
+    }
+    ConstItem* const itp = items + item;
+    ConstTask* const tp = tasks + itp->task;
+    const uint32_t node_start = itp->a, nrows = itp->b;
+    const uint32_t b = tp->bins;
+    float* const out = a.work +
+                       static_cast<uint64_t>((tp->regions >> tp->depth) & 1u) * a.nseries *
+                           plan.work_stride +
+                       sidx * plan.work_stride + tp->work_offset +
+                       static_cast<uint64_t>(node_start) * b;
+    const uint32_t c = node_regs_per_row(nrows, b);
+    if (c == 0) {
+      // generic: one level at a time between the two halves of the buffer
+      const uint32_t total = nrows * b;
+      const float* in = input_rows(itp, tp, sidx);
+      float* cur = lds;
+      float* nxt = lds + total;
+      __syncthreads();
+      for (uint32_t e = tid; e < total; e += kNodeThreads) cur[e] = in[e];
+      __syncthreads();
+      for (uint32_t d = tree_levels(nrows); d-- > 0;) {
+        for (uint32_t e = tid; e < total; e += kNodeThreads) {
+          const uint32_t r = e / b, p = e - r * b;
+          const Node nd = find_node(0, nrows, d, r);
+          float v = cur[e];
+          if (nd.size > 1) {
+            const Desc ds = merge_desc(nd, r, b);
+            uint32_t q = p + ds.roll;
+            q = min(q, q - b);
+            v = cur[ds.h * b + p] + cur[ds.t * b + q];
+          }
+          nxt[e] = v;
+        }
+        __syncthreads();
+        float* const t = cur;
+        cur = nxt;
+        nxt = t;
+      }
+      for (uint32_t e = tid; e < total; e += kNodeThreads) out[e] = cur[e];
+      continue;
+    }
+    {
+      uint32_t first;
+      const uint32_t n = sub_node(nrows, first);
+      const float* in = input_rows(itp, tp, sidx) + first * b;
+      with_regs_per_row(c, [&](auto cc) {
+        constexpr uint32_t C = decltype(cc)::value;
+        const int32_t p0 = static_cast<int32_t>(lane * C) - static_cast<int32_t>((C - b % C) % C);
+        run_sub_node<C>(n, in, lds + first * b, b, p0, node_start + first == 0);
+      });
+    }
+
+    // leaf j = lane % 8 of the rows 2 i, 2 i + 1 of the wave's pairs
+    // i = wave + 8 (lane / 8 + 8 m): its LDS offset (row * b + roll) and its
+    // combined roll (above bit 16); bits 8 q and 8 q + 4 of same[m]: the rows of
+    // pair slot q share their depth-1 head (tail) row
+    constexpr uint32_t kSets = (kNodeMaxRows / 2 + 8 * kNodeWaves - 1) / (8 * kNodeWaves);
+    uint32_t leaf[kSets][2];
+    uint64_t same[kSets];
+    {
+      // pick_row in integers (see below_row): the child row of row s is
+      // (s + up - (s > thr)) / 2, with the tail rolled by the rest of s
+      uint32_t start = 0, size = nrows;
+      uint32_t up[3], thr[3], rolled[3];
+#pragma unroll
+      for (uint32_t k = 0; k < 3; ++k) {
+        const bool tail = (lane >> (2 - k)) & 1u;
+        const uint32_t h = size / 2, odd = size & 1u;
+        up[k] = tail ? odd : 0u;
+        thr[k] = tail || !odd ? 0xFFFFu : h;
+        rolled[k] = tail ? 0xFFFFu : 0u;
+        start += tail ? h : 0u;
+        size = tail ? size - h : h;
+      }
+#pragma unroll
+      for (uint32_t m = 0; m < kSets; ++m) {
+        if (16 * kNodeWaves * m >= nrows) break;  // no pair in this set
+        uint32_t top[2];
+#pragma unroll
+        for (uint32_t v = 0; v < 2; ++v) {
+          uint32_t s = min(2 * (wave + kNodeWaves * ((lane >> 3) + 8 * m)) + v, nrows - 1);
+          uint32_t roll = 0;
+#pragma unroll
+          for (uint32_t k = 0; k < 3; ++k) {
+            const uint32_t t = (s + up[k] - (s > thr[k] ? 1u : 0u)) >> 1;
+            if (k == 0) top[v] = t;
+            roll += (s - t) & rolled[k];
+            s = t;
+          }
+          if (nrows > b) {  // a roll is below nrows <= 160, so below 3 b
+            roll = min(roll, roll - b);
+            roll = min(roll, roll - b);
+          }
+          leaf[m][v] = (__umul24(start + s, b) + roll) | (roll << 16);
+        }
+        same[m] = __ballot(top[0] == top[1]);
+      }
+    }
+    __syncthreads();
+    using LdsFloat = __attribute__((address_space(3))) const float;
+    LdsFloat* const rows = (LdsFloat*)lds;
+    const uint32_t nc = (b + 63) >> 6;
+    // v[p] = leaf (entry e)[(p + roll) mod b] for the row's chunks; chunks below
+    // NC - SEL cannot wrap, nor can leaf 0 (roll 0)
+    auto load_leaf = [&](auto ncv, auto selv, uint32_t e, bool rolled, float* v) {
+      constexpr uint32_t NC = decltype(ncv)::value;
+      constexpr uint32_t SEL = decltype(selv)::value < NC ? decltype(selv)::value : NC;
+      const uint32_t off = e & 0xFFFFu;
+      const uint32_t wrap = b - (e >> 16);  // phases before it do not wrap
+      LdsFloat* const ta = rows + off + lane;
+#pragma unroll
+      for (uint32_t k = 0; k < NC; ++k) {
+        if (k + SEL < NC || !rolled) {
+          v[k] = ta[64u * k];
+        } else {
+          const uint32_t x = off + lane + 64u * k;
+          v[k] = rows[lane + 64u * k < wrap ? x : x - b];
+        }
+      }
+    };
+    // output rows r and (where `two`) r + 1.  SH, ST: both read one depth-1 head
+    // (tail) row; the tail row is then read one phase further for row r + 1.
+    auto merge_pair = [&](auto ncv, auto selv, auto shv, auto stv, uint32_t r, uint32_t set,
+                          uint32_t slot, bool two) {
+      constexpr uint32_t NC = decltype(ncv)::value;
+      constexpr bool SH = decltype(shv)::value, ST = decltype(stv)::value;
+      float v[8][NC], w[8][NC];
+#pragma unroll
+      for (uint32_t j = 0; j < 8; ++j) {
+        load_leaf(ncv, selv, __builtin_amdgcn_readlane(leaf[set][0], slot * 8 + j), j != 0, v[j]);
+        if (j < 4 ? !SH : !ST)
+          load_leaf(ncv, selv, __builtin_amdgcn_readlane(leaf[set][1], slot * 8 + j), j != 0, w[j]);
+      }
+      auto half = [&](const float (&x)[8][NC], uint32_t j, uint32_t k) {
+        return (x[j][k] + x[j + 1][k]) + (x[j + 2][k] + x[j + 3][k]);
+      };
+      float* const o = out + r * b;
+      float tail[NC];
+#pragma unroll
+      for (uint32_t k = 0; k < NC; ++k) tail[k] = half(v, 4, k);
+#pragma unroll
+      for (uint32_t k = 0; k < NC; ++k) {
+        const float head = half(v, 0, k);
+        const uint32_t p = 64u * k + lane;
+        const bool in = k + 1 < NC || p < b;
+        // streaming: the next kernel reads the rows long after L2 could hold them
+        if (in) __builtin_nontemporal_store(head + tail[k], &o[p]);
+        if (two) {
+          const float h = SH ? head : half(w, 0, k);
+          float t;
+          if constexpr (ST) t = next_phase(tail[k], tail[(k + 1) % NC]);
+          else t = half(w, 4, k);
+          if (in) __builtin_nontemporal_store(h + t, &o[b + p]);
+        }
+      }
+    };
+    auto merge_rows = [&](auto ncv) {
+      constexpr uint32_t NC = decltype(ncv)::value;
+#pragma unroll
+      for (uint32_t m = 0; m < kSets; ++m) {
+        for (uint32_t q = 0; q < 8; ++q) {
+          const uint32_t r = 2 * (wave + kNodeWaves * (q + 8 * m));
+          if (r >= nrows) break;
+          const bool two = r + 1 < nrows;
+          auto with_sharing = [&](auto selv) {
+            const uint32_t bits = static_cast<uint32_t>(same[m] >> (8 * q)) & 0x11u;
+            if (bits == 0x11u) merge_pair(ncv, selv, std::true_type{}, std::true_type{}, r, m, q, two);
+            else if (bits == 0x01u) merge_pair(ncv, selv, std::true_type{}, std::false_type{}, r, m, q, two);
+            else if (bits == 0x10u) merge_pair(ncv, selv, std::false_type{}, std::true_type{}, r, m, q, two);
+            else merge_pair(ncv, selv, std::false_type{}, std::false_type{}, r, m, q, two);
+          };
+          if (r + 1 + 64u * (NC - 1) <= b) with_sharing(std::integral_constant<uint32_t, 1>{});
+          else if (NC > 2 && r + 1 + 64u * (NC - 2) <= b) with_sharing(std::integral_constant<uint32_t, 2>{});
+          else with_sharing(ncv);
+        }
+      }
+    };
+    static_assert(kNodeMinBins > 63 && kNodeMaxBins <= 320, "one case per chunk count");
+    if (nc == 4) merge_rows(std::integral_constant<uint32_t, 4>{});
+    else if (nc == 3) merge_rows(std::integral_constant<uint32_t, 3>{});
+    else if (nc == 5) merge_rows(std::integral_constant<uint32_t, 5>{});
+    else if (nc == 2) merge_rows(std::integral_constant<uint32_t, 2>{});
+    else merge_rows(std::integral_constant<uint32_t, 1>{});
   }
 }
 
@@ -1117,9 +1534,9 @@ namespace {
 // Raises a kernel's dynamic-LDS limit to at least `bytes`, never lowering
 // it: launches captured into a graph replay under the largest limit any of
 // them needed.  Per device and kernel (slot): subtree, detection, transform
-// rows, level.
+// rows, level, subtree in registers.
 void ensure_dynamic_lds(const void* kernel, int slot, uint32_t bytes) {
-  static uint32_t set[64][4] = {};
+  static uint32_t set[64][5] = {};
   int dev = 0;
   hip_check(hipGetDevice(&dev), "hipGetDevice");
   check(dev >= 0 && dev < 64, "device ordinal out of range");
@@ -1143,6 +1560,13 @@ int compute_units() {
     cus[dev] = n > 0 ? n : 1;
   }
   return cus[dev];
+}
+
+// Whether every node of the plan fits ffa_node_kernel.  Table sizes grow with
+// the rows, so the largest table bounds the rows of every node.
+bool nodes_in_registers(const gaffa_hip_ffa_plan_desc& p) {
+  static const uint32_t most = gaffa_hip_ffa_subtree_merges(kNodeMaxRows, 2, nullptr);
+  return p.max_bins <= kNodeMaxBins && p.max_subtree_desc <= most;
 }
 
 void launch_prepare(const gaffa_hip_ffa_search_args* a, hipStream_t st) {
@@ -1174,9 +1598,19 @@ void launch_subtrees(const gaffa_hip_ffa_search_args* a, hipStream_t st) {
   const gaffa_hip_ffa_plan_desc& p = *a->plan;
   const uint32_t ns = static_cast<uint32_t>(a->nseries);
   if (p.nsubtree_items > 0) {
-    ensure_dynamic_lds(reinterpret_cast<const void*>(ffa_subtree_kernel), 0, p.subtree_lds_bytes);
     const uint64_t nunits = static_cast<uint64_t>(p.nsubtree_items) * ns;
     check_overflow(nunits < (1ull << 32), "FFA subtree work too large");
+    if (nodes_in_registers(p)) {
+      const uint32_t bytes = node_lds_bytes(p.subtree_half_floats);
+      ensure_dynamic_lds(reinterpret_cast<const void*>(ffa_node_kernel), 4, bytes);
+      const uint32_t grid = static_cast<uint32_t>(
+          std::min<uint64_t>(nunits, 2ull * static_cast<uint64_t>(compute_units())));
+      hipLaunchKernelGGL(ffa_node_kernel, dim3(grid), dim3(kNodeThreads), bytes, st, kargs(a),
+                         static_cast<uint32_t>(nunits));
+      launch_check("ffa_node_kernel");
+      return;
+    }
+    ensure_dynamic_lds(reinterpret_cast<const void*>(ffa_subtree_kernel), 0, p.subtree_lds_bytes);
     // one resident workgroup per CU (the LDS footprint allows no more)
     const uint32_t grid = static_cast<uint32_t>(
         std::min<uint64_t>(nunits, static_cast<uint64_t>(compute_units())));
@@ -1284,7 +1718,10 @@ int gaffa_hip_ffa_reserve_launch(const gaffa_hip_ffa_plan_desc* p) {
     check(p->subtree_lds_bytes <= kMaxLdsBytes && p->terminal_lds_bytes <= kMaxLdsBytes &&
               p->level_lds_bytes <= kMaxLevelLdsBytes,
           "FFA plan exceeds LDS");
-    if (p->nsubtree_items > 0)
+    if (p->nsubtree_items > 0 && nodes_in_registers(*p))
+      ensure_dynamic_lds(reinterpret_cast<const void*>(ffa_node_kernel), 4,
+                         node_lds_bytes(p->subtree_half_floats));
+    else if (p->nsubtree_items > 0)
       ensure_dynamic_lds(reinterpret_cast<const void*>(ffa_subtree_kernel), 0,
                          p->subtree_lds_bytes);
     ensure_dynamic_lds(reinterpret_cast<const void*>(ffa_terminal_kernel<true>), 1,
