@@ -12,9 +12,11 @@
 //   detrend   - FP64 linear interpolation of the low-resolution median back to
 //               full resolution (same operation order as the CPU), subtract,
 //               write float
-//   stats     - one lane per series: the FP64 sum and sum of squares in
-//               sample order, exactly the CPU loop's roundings, then mean and
-//               1/stddev (time_series.cpp:50-77)
+//   stats     - the FP64 sum and sum of squares with exactly the roundings of
+//               the CPU loop, which adds in sample order, then mean and
+//               1/stddev (time_series.cpp:50-77): in parallel from maps of
+//               short runs, or, where the sum itself can round, a lane per
+//               series
 //   normalise - (x - mean) * (1/stddev) in FP64, rounded to float
 // Integer-valued inputs (dedispersed sums) make the scrunch sums exact, and
 // every other FP operation runs in the CPU's order, so the output is the
@@ -136,12 +138,30 @@ median_kernel(const T* __restrict__ src, uint64_t src_stride, uint64_t m,
   med[series * med_stride + static_cast<uint64_t>(k)] = value;
 }
 
-// x - interpolated median, written in place as float.
+// What the statistics need of one block of samples (see the statistics below).
+struct BlockSums {
+  double sum;        // of the samples, in any order
+  float squares;     // about the sum of squares
+  float magnitude;   // no less than the sum of |x|; inf or NaN where a sample is not finite
+  int32_t quantum;   // every sample is a multiple of 2^(quantum - 150)
+  int32_t exponent;  // block_exponent_kernel: the running sum of squares' exponent
+};
+
+// quantum of one sample: the exponent of its lowest set bit.
+__device__ __forceinline__ int32_t sample_quantum(float v) {
+  const uint32_t bits = __builtin_bit_cast(uint32_t, v) & 0x7FFFFFFFu;
+  const int32_t q = static_cast<int32_t>(max(bits >> 23, 1u)) + __builtin_ctz(bits | 0x800000u);
+  return bits == 0 ? 4096 : q;
+}
+
+// x - interpolated median, written in place as float; a workgroup runs
+// `items` x 256 samples and leaves their sums in sums[block] (where given).
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
 detrend_kernel(T* __restrict__ data, uint64_t stride, uint64_t n,
                int32_t detrend, uint64_t factor, const float* __restrict__ med,
-               uint64_t m, int32_t* __restrict__ status) {
+               uint64_t m, int32_t* __restrict__ status, uint32_t items,
+               BlockSums* __restrict__ sums) {
   const uint32_t tid = threadIdx.x;
   const uint64_t series = blockIdx.y;
   T* x = data + series * stride;
@@ -150,45 +170,211 @@ detrend_kernel(T* __restrict__ data, uint64_t stride, uint64_t n,
   const double offset = 0.5 * static_cast<double>(factor - 1);
   const double fd = static_cast<double>(factor);
   bool bad = false;
-  const uint64_t base = static_cast<uint64_t>(blockIdx.x) * kBlockSamples;
+  double sum = 0.0;
+  float squares = 0.0f, magnitude = 0.0f;
+  int32_t quantum = 4096;
+  const uint64_t base = static_cast<uint64_t>(blockIdx.x) * items * kThreads;
+  for (uint32_t r0 = 0; r0 < items; r0 += kDetrendItems) {
 #pragma unroll
-  for (int r = 0; r < kDetrendItems; ++r) {
-    const uint64_t i = base + static_cast<uint64_t>(r) * kThreads + tid;
-    if (i >= n) break;
-    const float v = load_as_float(x, i);
-    bad |= !isfinite(v);
-    float d = v;
-    if (detrend) {
-      float baseline;
-      if (factor == 1) {
-        baseline = md[i];
-      } else {
-        const double p = (static_cast<double>(i) - offset) / fd;
-        if (p <= 0.0) {
-          baseline = md[0];
+    for (int r = 0; r < kDetrendItems; ++r) {
+      const uint64_t i = base + static_cast<uint64_t>(r0 + r) * kThreads + tid;
+      if (i >= n) break;
+      const float v = load_as_float(x, i);
+      bad |= !isfinite(v);
+      float d = v;
+      if (detrend) {
+        float baseline;
+        if (factor == 1) {
+          baseline = md[i];
         } else {
-          const uint64_t lo = static_cast<uint64_t>(floor(p));
-          if (lo >= m - 1) {
-            baseline = md[m - 1];
+          const double p = (static_cast<double>(i) - offset) / fd;
+          if (p <= 0.0) {
+            baseline = md[0];
           } else {
-            const double fr = p - static_cast<double>(lo);
-            const double w0 = (1.0 - fr) * static_cast<double>(md[lo]);
-            const double w1 = fr * static_cast<double>(md[lo + 1]);
-            baseline = static_cast<float>(w0 + w1);
+            const uint64_t lo = static_cast<uint64_t>(floor(p));
+            if (lo >= m - 1) {
+              baseline = md[m - 1];
+            } else {
+              const double fr = p - static_cast<double>(lo);
+              const double w0 = (1.0 - fr) * static_cast<double>(md[lo]);
+              const double w1 = fr * static_cast<double>(md[lo + 1]);
+              baseline = static_cast<float>(w0 + w1);
+            }
           }
         }
+        d = v - baseline;
       }
-      d = v - baseline;
+      out[i] = d;
+      sum += static_cast<double>(d);
+      squares += d * d;
+      magnitude += fabsf(d);
+      quantum = min(quantum, sample_quantum(d));
     }
-    out[i] = d;
   }
   if (bad) atomicExch(&status[series], 1);
+  if (sums == nullptr) return;
+  __shared__ BlockSums part[kThreads / 64];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    sum += __shfl_xor(sum, off, 64);
+    squares += __shfl_xor(squares, off, 64);
+    magnitude += __shfl_xor(magnitude, off, 64);
+    quantum = min(quantum, __shfl_xor(quantum, off, 64));
+  }
+  if ((tid & 63u) == 0) part[tid >> 6] = BlockSums{sum, squares, magnitude, quantum, 0};
+  __syncthreads();
+  if (tid == 0) {
+    BlockSums t = part[0];
+    for (int w = 1; w < kThreads / 64; ++w) {
+      t.sum += part[w].sum;
+      t.squares += part[w].squares;
+      t.magnitude += part[w].magnitude;
+      t.quantum = min(t.quantum, part[w].quantum);
+    }
+    t.magnitude *= 1.01f;  // past the rounding of its float sum
+    sums[series * gridDim.x + blockIdx.x] = t;
+  }
 }
 
-// Sum and sum of squares of each series in FP64 in sample order, as
-// time_series_stats_cpu does (time_series.cpp:55-60), so every rounding is
-// the CPU's; then mean, 1/stddev and a status flag.
+// Statistics: the sum and sum of squares of each series in FP64 in sample order,
+// as time_series_stats_cpu does (time_series.cpp:55-60), so every rounding is the
+// CPU's; then mean, 1/stddev and a status flag.
 //
+// One FP64 add per sample and chain is a chain of n dependent adds, whatever the
+// batch: 12 ns a sample in stats_kernel, 12.7 ms at 2^20 samples.  Both sums can
+// be had in parallel with the same bits:
+//   sum      where every sample is a multiple of some 2^q and the sum of |x| is
+//            below 2^53 2^q, no partial sum rounds, in any order.  Detrended
+//            integer series are such: x is a difference of multiples of the
+//            baseline's last place.
+//   squares  the running sum S never falls.  While it stays in one binade
+//            [2^k, 2^(k+1)), with last place u, adding q rounds to S + m u where m
+//            depends on q and, in a tie, on the parity of S / u alone.  So a run
+//            of samples maps a parity to an increment, and such maps compose in
+//            any grouping.  Each thread measures its run's two increments by
+//            adding it to 2^k and to 2^k + u, with the real FP64 adds.
+// detrend_kernel leaves each block's sums, block_exponent_kernel predicts k for
+// every block from their prefix sums, square_map_kernel composes each block's
+// map, and combine_stats_kernel walks the blocks of a series: it applies a map
+// only where S really starts and ends in the map's binade, and else runs the
+// block in finer pieces, down to sample by sample around a binade's end.  Series
+// whose sum can round (or with a sample that is not finite) are left to
+// stats_kernel.
+// The read of the plane bounds square_map_kernel.  Measured, statistics with
+// their part of detrend_kernel: 256 series of 2^20 samples 12.7 -> 0.5 ms, 512
+// of 2^21 25.1 -> 1.2 ms, 128 of 400k 4.8 -> 0.2 ms.
+constexpr uint32_t kMapThreads = 512;
+constexpr uint32_t kMapRun = 8;                           // samples per thread and step
+constexpr uint32_t kMapBlock = kMapThreads * kMapRun;     // smallest block: 4096 samples
+constexpr uint32_t kMapMaxShift = 4;                      // blocks of up to 65536 samples
+constexpr int32_t kNoExponent = -1;                       // a block that holds a binade's end
+constexpr int32_t kZeroBlock = -2;                        // a block of zeros
+constexpr int32_t kSerialStats = -1;                      // flags: left to stats_kernel
+
+// The biased exponent of x >= 0 (zero for a zero).
+__device__ __forceinline__ int32_t exponent_of(double x) {
+  return static_cast<int32_t>(__builtin_bit_cast(uint64_t, x) >> 52);
+}
+__device__ __forceinline__ double binade(int32_t exponent) {
+  return __builtin_bit_cast(double, static_cast<uint64_t>(exponent) << 52);
+}
+__device__ __forceinline__ bool is_odd(double x) {
+  return (__builtin_bit_cast(uint64_t, x) & 1u) != 0;
+}
+// The exponent that a running sum from `from` to `to` (both about right) keeps.
+__device__ __forceinline__ int32_t kept_exponent(double from, double to, double margin) {
+  const int32_t lo = exponent_of(from * (1.0 - margin)), hi = exponent_of(to * (1.0 + margin));
+  return lo == hi && lo > 53 && hi < 0x7FE ? lo : kNoExponent;
+}
+
+// A run's increments of a sum in binade k that starts even (x) or odd (y).
+__device__ __forceinline__ double2 compose(double2 f, double2 g, double base) {
+  return make_double2(f.x + (is_odd(base + f.x) ? g.y : g.x),
+                      f.y + (is_odd(base + f.y) ? g.x : g.y));
+}
+
+__device__ __forceinline__ double read_lane(double x, uint32_t lane) {
+  const uint64_t bits = __builtin_bit_cast(uint64_t, x);
+  const uint64_t lo = static_cast<uint32_t>(
+      __builtin_amdgcn_readlane(static_cast<int>(bits), static_cast<int>(lane)));
+  const uint64_t hi = static_cast<uint32_t>(
+      __builtin_amdgcn_readlane(static_cast<int>(bits >> 32), static_cast<int>(lane)));
+  return __builtin_bit_cast(double, lo | (hi << 32));
+}
+
+// sums[b].exponent of every block of a series, a wave per series.
+__global__ void __launch_bounds__(64)
+block_exponent_kernel(BlockSums* __restrict__ sums, uint32_t nblocks) {
+  BlockSums* const s = sums + static_cast<uint64_t>(blockIdx.x) * nblocks;
+  const uint32_t lane = threadIdx.x;
+  double before = 0.0;
+  for (uint32_t b0 = 0; b0 < nblocks; b0 += 64) {
+    const uint32_t b = b0 + lane;
+    const double q = b < nblocks ? static_cast<double>(s[b].squares) : 0.0;
+    double upto = q;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const double x = __shfl_up(upto, off, 64);
+      if (lane >= static_cast<uint32_t>(off)) upto += x;
+    }
+    if (b < nblocks)
+      s[b].exponent = kept_exponent(before + (upto - q), before + upto, 1e-5);
+    before += read_lane(upto, 63);
+  }
+}
+
+// maps[series][block]: the block's increments of the sum of squares.
+__global__ void __launch_bounds__(kMapThreads)
+square_map_kernel(const float* __restrict__ data, uint64_t stride, uint64_t n, uint32_t run,
+                  const BlockSums* __restrict__ sums, double2* __restrict__ maps) {
+  const uint64_t block = static_cast<uint64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
+  const int32_t k = sums[block].exponent;
+  if (k < 0) return;
+  const float* x = data + blockIdx.y * stride;
+  const uint32_t tid = threadIdx.x;
+  const uint64_t i0 = (static_cast<uint64_t>(blockIdx.x) * kMapThreads + tid) * run;
+  const double base = binade(k);
+  const double odd = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, base) | 1u);
+  double a = base, c = odd;
+  struct Run {
+    float x[kMapRun];
+  };
+  for (uint32_t r = 0; r < run; r += kMapRun) {
+    const uint64_t i = i0 + r;
+    if (i + kMapRun <= n) {
+      const Run v = *reinterpret_cast<const Run*>(x + i);
+#pragma unroll
+      for (uint32_t u = 0; u < kMapRun; ++u) {
+        const double d = static_cast<double>(v.x[u]);
+        const double q = d * d;
+        a = a + q;
+        c = c + q;
+      }
+    } else {
+      for (uint64_t e = i; e < n; ++e) {
+        const double d = static_cast<double>(x[e]);
+        const double q = d * d;
+        a = a + q;
+        c = c + q;
+      }
+    }
+  }
+  double2 f = make_double2(a - base, c - odd);
+  // runs in order: lane l joins lane l + off, for growing off
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const double2 g = make_double2(__shfl_down(f.x, off, 64), __shfl_down(f.y, off, 64));
+    f = compose(f, g, base);  // lanes that are not a multiple of 2 off are not read again
+  }
+  __shared__ double2 part[kMapThreads / 64];
+  if ((tid & 63u) == 0) part[tid >> 6] = f;
+  __syncthreads();
+  if (tid == 0) {
+    for (uint32_t w = 1; w < kMapThreads / 64; ++w) f = compose(f, part[w], base);
+    maps[block] = f;
+  }
+}
+
 // A two-wave workgroup owns 64 series, a lane of each wave per series: wave 0
 // runs the chain of sums, wave 1 the chain of squares (the two are
 // independent, so each wave has one serial chain instead of two and the
@@ -224,6 +410,16 @@ struct SerialSums {
   }
 };
 
+// Whether S plus a map's increment is what the adds give: it starts and ends in
+// binade k.  Then S becomes it.
+__device__ __forceinline__ bool apply_map(double& S, int32_t k, double even, double odd) {
+  if (k < 0 || exponent_of(S) != k) return false;
+  const double to = S + (is_odd(S) ? odd : even);
+  if (exponent_of(to) != k) return false;
+  S = to;
+  return true;
+}
+
 __device__ __forceinline__ void finish_stats(const SerialSums& acc, uint64_t n, uint32_t series,
                                              int32_t reject_constant, double2* stats,
                                              int32_t* flags, int32_t* status) {
@@ -240,10 +436,110 @@ __device__ __forceinline__ void finish_stats(const SerialSums& acc, uint64_t n, 
   if (flag == 2 || flag == 3) atomicCAS(&status[series], 0, flag);
 }
 
+// One wave per series: S over the blocks' maps, finer where a map does not hold.
+__global__ void __launch_bounds__(64)
+combine_stats_kernel(const float* __restrict__ data, uint64_t stride, uint64_t n,
+                     uint32_t nblocks, uint32_t block, const BlockSums* __restrict__ sums,
+                     const double2* __restrict__ maps, int32_t reject_constant,
+                     double2* __restrict__ stats, int32_t* __restrict__ flags,
+                     int32_t* __restrict__ status) {
+  const uint32_t series = blockIdx.x;
+  const uint32_t lane = threadIdx.x;
+  const float* x = data + series * stride;
+  const BlockSums* const s = sums + static_cast<uint64_t>(series) * nblocks;
+  const double2* const f = maps + static_cast<uint64_t>(series) * nblocks;
+  SerialSums acc;
+  double magnitude = 0.0;
+  int32_t quantum = 4096;
+  for (uint32_t b = lane; b < nblocks; b += 64) {
+    acc.sum += s[b].sum;
+    magnitude += static_cast<double>(s[b].magnitude);
+    quantum = min(quantum, s[b].quantum);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    acc.sum += __shfl_xor(acc.sum, off, 64);
+    magnitude += __shfl_xor(magnitude, off, 64);
+    quantum = min(quantum, __shfl_xor(quantum, off, 64));
+  }
+  // multiples of 2^(quantum - 150) that add up to less than 2^53 of them
+  if (!(magnitude < ldexp(1.0, min(quantum, 400) - 150 + 52))) {
+    if (lane == 0) flags[series] = kSerialStats;
+    return;
+  }
+  constexpr uint32_t kRun = 32;  // samples per lane in a block run in finer pieces
+  double S = 0.0;
+  for (uint32_t b0 = 0; b0 < nblocks; b0 += 64) {
+    const uint32_t b = b0 + lane;
+    int32_t k = kZeroBlock;
+    double2 map = make_double2(0.0, 0.0);
+    if (b < nblocks) {
+      k = s[b].magnitude == 0.0f ? kZeroBlock : s[b].exponent;
+      if (k >= 0) map = f[b];
+    }
+    const uint32_t count = min(64u, nblocks - b0);
+    for (uint32_t l = 0; l < count; ++l) {
+      const int32_t kl = __builtin_amdgcn_readlane(k, l);
+      if (kl == kZeroBlock) continue;  // adding zeros leaves S as it is
+      if (apply_map(S, kl, read_lane(map.x, l), read_lane(map.y, l))) continue;
+      const uint64_t first = static_cast<uint64_t>(b0 + l) * block;
+      const uint64_t last = min(n, first + block);
+      for (uint64_t p = first; p < last; p += 64 * kRun) {
+        float v[kRun];
+        double own = 0.0;
+#pragma unroll
+        for (uint32_t j = 0; j < kRun; ++j) {
+          const uint64_t i = p + lane * kRun + j;
+          v[j] = i < last ? x[i] : 0.0f;
+          own += static_cast<double>(v[j]) * static_cast<double>(v[j]);
+        }
+        double upto = own;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const double y = __shfl_up(upto, off, 64);
+          if (lane >= static_cast<uint32_t>(off)) upto += y;
+        }
+        const int32_t kr = kept_exponent(S + (upto - own), S + upto, 1e-9);
+        const double base = binade(max(kr, 0));
+        const double odd = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, base) | 1u);
+        double a = base, c = odd;
+#pragma unroll
+        for (uint32_t j = 0; j < kRun; ++j) {
+          const double q = static_cast<double>(v[j]) * static_cast<double>(v[j]);
+          a = a + q;
+          c = c + q;
+        }
+        a -= base;
+        c -= odd;
+        for (uint32_t w = 0; w < 64; ++w) {
+          if (apply_map(S, __builtin_amdgcn_readlane(kr, w), read_lane(a, w), read_lane(c, w)))
+            continue;
+#pragma unroll
+          for (uint32_t j = 0; j < kRun; ++j) {
+            const double d = static_cast<double>(__builtin_bit_cast(
+                float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[j]), w)));
+            S = S + d * d;
+          }
+        }
+      }
+    }
+  }
+  acc.squares = S;
+  if (lane == 0) finish_stats(acc, n, series, reject_constant, stats, flags, status);
+}
+
+// Whether any of the workgroup's series was left to it (`flagged`: the launch
+// follows combine_stats_kernel; else every series is).
+__device__ __forceinline__ bool any_serial(const int32_t* flags, uint32_t first, uint32_t rows,
+                                           bool flagged) {
+  const uint32_t lane = threadIdx.x & 63u;
+  return !flagged || __ballot(lane < rows && flags[first + lane] == kSerialStats) != 0;
+}
+
 __global__ void __launch_bounds__(kStatsThreads) __attribute__((amdgpu_waves_per_eu(1, 2)))
 stats_kernel(const float* __restrict__ data, uint64_t stride, uint64_t n, uint32_t nseries,
              int32_t reject_constant, double2* __restrict__ stats,
-             int32_t* __restrict__ flags, int32_t* __restrict__ status) {
+             int32_t* __restrict__ flags, int32_t* __restrict__ status, bool flagged) {
   extern __shared__ __align__(16) float stage[];  // [2][kStatsLanes][kStatsPitch]
   __shared__ double squares_of[kStatsLanes];
   const uint32_t tid = threadIdx.x;
@@ -251,6 +547,7 @@ stats_kernel(const float* __restrict__ data, uint64_t stride, uint64_t n, uint32
   const bool squares = tid >= 64u;  // wave-uniform: wave 1 runs the squares
   const uint32_t first = blockIdx.x * kStatsLanes;
   const uint32_t rows = min(static_cast<uint32_t>(kStatsLanes), nseries - first);
+  if (!any_serial(flags, first, rows, flagged)) return;
   const uint64_t nchunks = n / kStatsChunk;
   const float* base = data + static_cast<uint64_t>(first) * stride;
   // load k of a chunk: element e = k * 128 + tid is row e / kStatsVecs,
@@ -342,8 +639,11 @@ stats_kernel(const float* __restrict__ data, uint64_t stride, uint64_t n, uint32
 __global__ void __launch_bounds__(kStatsLanes)
 stats_rowwise_kernel(const float* __restrict__ data, uint64_t stride, uint64_t n,
                      uint32_t nseries, int32_t reject_constant, double2* __restrict__ stats,
-                     int32_t* __restrict__ flags, int32_t* __restrict__ status) {
-  const uint32_t series = blockIdx.x * kStatsLanes + threadIdx.x;
+                     int32_t* __restrict__ flags, int32_t* __restrict__ status, bool flagged) {
+  const uint32_t first = blockIdx.x * kStatsLanes;
+  const uint32_t series = first + threadIdx.x;
+  if (!any_serial(flags, first, min(static_cast<uint32_t>(kStatsLanes), nseries - first), flagged))
+    return;
   if (series >= nseries) return;
   const float* x = data + static_cast<uint64_t>(series) * stride;
   SerialSums acc;
@@ -411,6 +711,42 @@ Layout layout(uint64_t nseries, uint64_t n, uint64_t factor) {
   return l;
 }
 
+// Where the parallel statistics keep their blocks: the low-resolution series is
+// free once its medians are taken, and the medians once they are subtracted, so
+// blocks of kMapBlock << shift samples live there and need no room of their own.
+// Off where they do not fit (scrunch factors past 10^4, an exact running median,
+// which leaves no low-resolution series): stats_kernel then runs every series.
+struct StatsBlocks {
+  bool on = false;
+  uint32_t shift = 0;
+  uint64_t nblocks = 0;
+  BlockSums* sums = nullptr;
+  double2* maps = nullptr;
+};
+
+StatsBlocks stats_blocks(const gaffa_hip_preprocess_args* a, const Layout& l, void* workspace) {
+  StatsBlocks s;
+  if (!a->normalise || (a->detrend && a->scrunch_factor == 1)) return s;
+  auto align = [](uint64_t v) { return (v + 15) / 16 * 16; };
+  const uint64_t end = (l.low_floats + l.med_floats) * 4;
+  for (uint32_t shift = 0; shift <= kMapMaxShift; ++shift) {
+    const uint64_t nblocks = ceil_div(a->nsamples, static_cast<uint64_t>(kMapBlock) << shift);
+    const uint64_t sums = a->nseries * nblocks * sizeof(BlockSums);
+    // the detrend pass reads the medians while it writes the sums
+    const uint64_t maps = align(a->detrend ? l.low_floats * 4 : sums);
+    if ((a->detrend && sums > l.low_floats * 4) ||
+        maps + a->nseries * nblocks * sizeof(double2) > end)
+      continue;
+    s.on = true;
+    s.shift = shift;
+    s.nblocks = nblocks;
+    s.sums = static_cast<BlockSums*>(workspace);
+    s.maps = reinterpret_cast<double2*>(static_cast<char*>(workspace) + maps);
+    return s;
+  }
+  return s;
+}
+
 template <typename T>
 void run(const gaffa_hip_preprocess_args* a, void* workspace, hipStream_t st) {
   const Layout l = layout(a->nseries, a->nsamples, a->detrend ? a->scrunch_factor : 1);
@@ -443,12 +779,30 @@ void run(const gaffa_hip_preprocess_args* a, void* workspace, hipStream_t st) {
     }
   }
   const dim3 g(static_cast<uint32_t>(l.nblocks), static_cast<uint32_t>(a->nseries));
-  hipLaunchKernelGGL((detrend_kernel<T>), g, dim3(kThreads), 0, st, data, a->stride, a->nsamples,
-                     a->detrend, a->detrend ? f : 1, med, l.m, a->status);
+  const StatsBlocks sb = stats_blocks(a, l, workspace);
+  const uint32_t block = kMapBlock << sb.shift;
+  const dim3 dg(static_cast<uint32_t>(sb.on ? sb.nblocks : l.nblocks),
+                static_cast<uint32_t>(a->nseries));
+  hipLaunchKernelGGL((detrend_kernel<T>), dg, dim3(kThreads), 0, st, data, a->stride, a->nsamples,
+                     a->detrend, a->detrend ? f : 1, med, l.m, a->status,
+                     sb.on ? block / kThreads : static_cast<uint32_t>(kDetrendItems), sb.sums);
   launch_check("detrend_kernel");
   if (a->normalise) {
     const dim3 sg(static_cast<uint32_t>(ceil_div(a->nseries, kStatsLanes)));
     const float* fdata = reinterpret_cast<const float*>(data);
+    if (sb.on) {
+      const uint32_t ns = static_cast<uint32_t>(a->nseries);
+      const uint32_t nblocks = static_cast<uint32_t>(sb.nblocks);
+      hipLaunchKernelGGL(block_exponent_kernel, dim3(ns), dim3(64), 0, st, sb.sums, nblocks);
+      launch_check("block_exponent_kernel");
+      hipLaunchKernelGGL(square_map_kernel, dim3(nblocks, ns), dim3(kMapThreads), 0, st, fdata,
+                         a->stride, a->nsamples, block / kMapThreads, sb.sums, sb.maps);
+      launch_check("square_map_kernel");
+      hipLaunchKernelGGL(combine_stats_kernel, dim3(ns), dim3(64), 0, st, fdata, a->stride,
+                         a->nsamples, nblocks, block, sb.sums, sb.maps, a->reject_constant, stats,
+                         flags, a->status);
+      launch_check("combine_stats_kernel");
+    }
     if ((reinterpret_cast<uintptr_t>(fdata) & 15u) == 0 && a->stride % 4 == 0) {
       // two chunk buffers exceed the default 64 KiB of dynamic LDS
       hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(stats_kernel),
@@ -457,12 +811,12 @@ void run(const gaffa_hip_preprocess_args* a, void* workspace, hipStream_t st) {
                 "hipFuncSetAttribute");
       hipLaunchKernelGGL(stats_kernel, sg, dim3(kStatsThreads), kStatsLdsBytes, st, fdata,
                          a->stride, a->nsamples, static_cast<uint32_t>(a->nseries),
-                         a->reject_constant, stats, flags, a->status);
+                         a->reject_constant, stats, flags, a->status, sb.on);
       launch_check("stats_kernel");
     } else {
       hipLaunchKernelGGL(stats_rowwise_kernel, sg, dim3(kStatsLanes), 0, st, fdata, a->stride,
                          a->nsamples, static_cast<uint32_t>(a->nseries), a->reject_constant,
-                         stats, flags, a->status);
+                         stats, flags, a->status, sb.on);
       launch_check("stats_rowwise_kernel");
     }
     hipLaunchKernelGGL(normalise_kernel, g, dim3(kThreads), 0, st,

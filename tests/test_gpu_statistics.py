@@ -1,0 +1,96 @@
+"""GPU parity of the FP64 statistics with sums in sample order, bit for bit."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+class PreprocessArgs(ctypes.Structure):
+    _fields_ = [("data", ctypes.c_void_p), ("nseries", ctypes.c_uint64),
+                ("nsamples", ctypes.c_uint64), ("stride", ctypes.c_uint64),
+                ("input_is_u32", ctypes.c_int32), ("detrend", ctypes.c_int32),
+                ("scrunch_factor", ctypes.c_uint64), ("median_window", ctypes.c_uint64),
+                ("normalise", ctypes.c_int32), ("reject_constant", ctypes.c_int32),
+                ("workspace", ctypes.c_void_p), ("workspace_bytes", ctypes.c_uint64),
+                ("status", ctypes.c_void_p)]
+
+
+def _series(kind, n, rng):
+    if kind == "integers":       # exact sums, squares that round once they are large
+        return np.rint(rng.normal(0.0, 300.0, n))
+    if kind == "tenths":         # multiples of 2^-10, as detrended series: half the adds tie
+        return np.rint(rng.normal(0.0, 90.0, n) * 1024.0) / 1024.0
+    if kind == "bursts":         # the sum of squares crosses binades inside blocks
+        x = np.rint(rng.normal(0.0, 2.0, n))
+        x[rng.integers(0, n, 12)] = 2.0 ** rng.integers(3, 19, 12)
+        return x
+    if kind == "late":           # zeros, then one sample, then noise
+        x = np.rint(rng.normal(0.0, 50.0, n))
+        x[: 2 * n // 3] = 0.0
+        x[n // 3] = 7.0
+        return x
+    if kind == "tiny":           # squares below the float range
+        return np.rint(rng.normal(0.0, 50.0, n)) * 2.0 ** -100
+    return rng.normal(0.0, 1.0, n)  # "floats": the sum itself rounds
+
+
+def _statistics(x, factor, stride):
+    """(mean, 1/sigma) the library leaves in its workspace, per series."""
+    import gaffa_amd
+
+    lib = ctypes.CDLL(gaffa_amd.HIP_LIBRARY)
+    f = lib.gaffa_hip_preprocess_workspace_bytes
+    f.restype, f.argtypes = ctypes.c_uint64, [ctypes.c_uint64] * 3
+    ns, n = x.shape
+    rows = np.zeros((ns, stride), np.float32)
+    rows[:, :n] = x
+    need = f(ns, n, factor)
+    ptrs = []
+
+    def dev(nbytes):
+        p = ctypes.c_void_p()
+        assert lib.gaffa_hip_malloc(ctypes.byref(p), ctypes.c_uint64(nbytes)) == 0
+        ptrs.append(p)
+        return p
+
+    def copy(dst, src, nbytes):
+        assert lib.gaffa_hip_memcpy(dst, src, ctypes.c_uint64(nbytes), None) == 0
+
+    try:
+        d, st, ws = dev(rows.nbytes), dev(4 * ns), dev(need)
+        copy(d, rows.ctypes.data_as(ctypes.c_void_p), rows.nbytes)
+        assert lib.gaffa_hip_memset(st, 0, ctypes.c_uint64(4 * ns), None) == 0
+        a = PreprocessArgs(d, ns, n, stride, 0, 0, 1, 1, 1, 1, ws, need, st)
+        assert lib.gaffa_hip_detrend_normalise_batch(ctypes.byref(a), None) == 0
+        assert lib.gaffa_hip_device_synchronize() == 0
+        # the scratch of n floats a series, then the statistics
+        at = (ns * n * 4 + 255) // 256 * 256
+        out = np.empty((ns, 2), np.float64)
+        copy(out.ctypes.data_as(ctypes.c_void_p), ctypes.c_void_p(ws.value + at), out.nbytes)
+        return out
+    finally:
+        for p in ptrs:
+            lib.gaffa_hip_free(p)
+
+
+@pytest.mark.parametrize("kind", ["integers", "tenths", "bursts", "late", "tiny", "floats"])
+def test_statistics_equal_sums_in_sample_order(gpu, kind):
+    """Mean and 1/sigma of every series equal the FP64 sums in sample order bit
+    for bit, around the block (4096) and run sizes, over binade crossings, and
+    where the plain sum rounds (the serial chain); aligned rows and rows that
+    are not."""
+    rng = np.random.default_rng(len(kind))
+    for ns, n, stride in ((3, 2, 4), (2, 31, 31), (66, 4095, 4096), (3, 4096, 4096),
+                          (5, 4097, 4099), (2, 70001, 70001), (3, 300000, 300032)):
+        print(f"statistics: {kind}, {ns} series x {n} (stride {stride})", flush=True)
+        x = np.stack([_series(kind, n, rng) for _ in range(ns)]).astype(np.float32)
+        x[:, 0] += 1.0  # never constant
+        got = _statistics(x, 1, stride)
+        d = x.astype(np.float64)
+        mean = np.cumsum(d, axis=1)[:, -1] / n
+        var = np.cumsum(d * d, axis=1)[:, -1] / n - mean * mean
+        np.testing.assert_array_equal(got[:, 0], mean)
+        np.testing.assert_array_equal(got[:, 1], 1.0 / np.sqrt(var))
