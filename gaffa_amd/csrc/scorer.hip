@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace gaffa_hip {
 namespace {
@@ -53,12 +54,67 @@ __device__ __forceinline__ void gemm_store(const gaffa_hip_gemm_args& g, uint32_
   if (g.c16 != nullptr) g.c16[o] = to_bf16(v);
 }
 
+// How a 64 x 32 operand tile is read, 8 values per thread in one 16-byte load:
+// along k, along the operand's other index (its values then go to LDS one by
+// one), or value by value where neither is contiguous and aligned.
+enum class Load { kK, kOther, kScalar };
+
+// One operand's tile: rows `first` .. + 63 of `rows`, columns k0 .. + 31 below
+// `k_end`; element (i, k) at p[i * row + k * col], 0 outside.
+template <Load kMode>
+struct Tile {
+  union {
+    uint4 vec;
+    uint16_t v[8];
+  };
+
+  __device__ __forceinline__ void load(const uint16_t* p, int64_t row, int64_t col, uint32_t first,
+                                       uint32_t rows, uint32_t k0, uint32_t k_end, uint32_t t) {
+    vec = make_uint4(0, 0, 0, 0);
+    if constexpr (kMode == Load::kK) {
+      const uint32_t i = first + (t >> 2), k = k0 + (t & 3u) * 8u;
+      if (i < rows && k < k_end)
+        vec = *reinterpret_cast<const uint4*>(p + static_cast<int64_t>(i) * row + k);
+    } else if constexpr (kMode == Load::kOther) {
+      const uint32_t i = first + (t & 7u) * 8u, k = k0 + (t >> 3);
+      if (i < rows && k < k_end)
+        vec = *reinterpret_cast<const uint4*>(p + static_cast<int64_t>(k) * col + i);
+    } else {
+      const bool i_fast = row == 1;
+      for (uint32_t q = 0; q < 8; ++q) {
+        const uint32_t e = t + 256u * q;
+        const uint32_t i = first + (i_fast ? e % kBM : e / kBK);
+        const uint32_t k = k0 + (i_fast ? e / kBM : e % kBK);
+        if (i < rows && k < k_end)
+          v[q] = p[static_cast<int64_t>(i) * row + static_cast<int64_t>(k) * col];
+      }
+    }
+  }
+
+  __device__ __forceinline__ void store(uint16_t* lds, int64_t row, uint32_t t) const {
+    if constexpr (kMode == Load::kK) {
+      *reinterpret_cast<uint4*>(&lds[(t >> 2) * kLdsK + (t & 3u) * 8u]) = vec;
+    } else if constexpr (kMode == Load::kOther) {
+#pragma unroll
+      for (uint32_t q = 0; q < 8; ++q) lds[((t & 7u) * 8u + q) * kLdsK + (t >> 3)] = v[q];
+    } else {
+      const bool i_fast = row == 1;
+      for (uint32_t q = 0; q < 8; ++q) {
+        const uint32_t e = t + 256u * q;
+        lds[(i_fast ? e % kBM : e / kBK) * kLdsK + (i_fast ? e / kBM : e % kBK)] = v[q];
+      }
+    }
+  }
+};
+
 // 64 x 64 output tile per workgroup, four waves of 32 x 32 (2 x 2 MFMA
 // blocks).  Operand fragments, per lane l of a 16 x 16 x 32 block: A row
 // l % 16, k = 8 (l / 16) .. + 7; B column l % 16, the same k; result rows
-// 4 (l / 16) .. + 3 of column l % 16.  kAFast: A is K-contiguous (a_col 1,
-// a_row and the base 16-byte aligned); kBFast: B is K-contiguous (b_row 1).
-template <bool kAFast, bool kBFast>
+// 4 (l / 16) .. + 3 of column l % 16.  The next tiles are in flight while the
+// current ones multiply: a weight gradient (64 x 192 over 32576 batch rows in 31
+// splits) has 93 workgroups, so the latency of a step's loads is its time, 115 us
+// with 16 two-byte loads per thread and step and none in flight, 37 us now.
+template <Load kA, Load kB>
 __global__ void __launch_bounds__(256) gemm_kernel(gaffa_hip_gemm_args g, uint32_t kchunk) {
   __shared__ __attribute__((aligned(16))) uint16_t as[kBM * kLdsK];
   __shared__ __attribute__((aligned(16))) uint16_t bs[kBN * kLdsK];
@@ -71,42 +127,16 @@ __global__ void __launch_bounds__(256) gemm_kernel(gaffa_hip_gemm_args g, uint32
   for (int x = 0; x < 2; ++x)
     for (int y = 0; y < 2; ++y) acc[x][y] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
+  Tile<kA> ta;
+  Tile<kB> tb;
+  ta.load(g.a, g.a_row, g.a_col, i0, g.m, kb, ke, t);
+  tb.load(g.b, g.b_col, g.b_row, j0, g.n, kb, ke, t);
   for (uint32_t k0 = kb; k0 < ke; k0 += kBK) {
-    if constexpr (kAFast) {
-      const uint32_t i = t >> 2, kk = (t & 3u) * 8u;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (i0 + i < g.m && k0 + kk < ke)
-        v = *reinterpret_cast<const uint4*>(g.a + static_cast<int64_t>(i0 + i) * g.a_row + k0 + kk);
-      *reinterpret_cast<uint4*>(&as[i * kLdsK + kk]) = v;
-    } else {
-      const bool i_fast = g.a_row == 1;
-      for (uint32_t q = 0; q < 8; ++q) {
-        const uint32_t e = t + 256u * q;
-        const uint32_t i = i_fast ? e % kBM : e / kBK;
-        const uint32_t kk = i_fast ? e / kBM : e % kBK;
-        uint16_t v = 0;
-        if (i0 + i < g.m && k0 + kk < ke)
-          v = g.a[static_cast<int64_t>(i0 + i) * g.a_row + static_cast<int64_t>(k0 + kk) * g.a_col];
-        as[i * kLdsK + kk] = v;
-      }
-    }
-    if constexpr (kBFast) {
-      const uint32_t j = t >> 2, kk = (t & 3u) * 8u;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (j0 + j < g.n && k0 + kk < ke)
-        v = *reinterpret_cast<const uint4*>(g.b + static_cast<int64_t>(j0 + j) * g.b_col + k0 + kk);
-      *reinterpret_cast<uint4*>(&bs[j * kLdsK + kk]) = v;
-    } else {
-      const bool j_fast = g.b_col == 1;
-      for (uint32_t q = 0; q < 8; ++q) {
-        const uint32_t e = t + 256u * q;
-        const uint32_t j = j_fast ? e % kBN : e / kBK;
-        const uint32_t kk = j_fast ? e / kBN : e % kBK;
-        uint16_t v = 0;
-        if (j0 + j < g.n && k0 + kk < ke)
-          v = g.b[static_cast<int64_t>(k0 + kk) * g.b_row + static_cast<int64_t>(j0 + j) * g.b_col];
-        bs[j * kLdsK + kk] = v;
-      }
+    ta.store(as, g.a_row, t);
+    tb.store(bs, g.b_col, t);
+    if (k0 + kBK < ke) {
+      ta.load(g.a, g.a_row, g.a_col, i0, g.m, k0 + kBK, ke, t);
+      tb.load(g.b, g.b_col, g.b_row, j0, g.n, k0 + kBK, ke, t);
     }
     __syncthreads();
     bf16x8 af[2], bf[2];
@@ -163,18 +193,27 @@ void launch_gemm(const gaffa_hip_gemm_args& g, hipStream_t st) {
   const uint32_t splits = static_cast<uint32_t>(ceil_div(g.k, kchunk));
   gaffa_hip_gemm_args a = g;
   a.k_splits = splits;
-  const bool af = g.a_col == 1 && g.a_row % 8 == 0 && g.k % 8 == 0 && aligned16(g.a);
-  const bool bf = g.b_row == 1 && g.b_col % 8 == 0 && g.k % 8 == 0 && aligned16(g.b);
+  // 16-byte loads need the tile's run of 8 values inside the operand and aligned
+  const auto mode = [&](const uint16_t* p, int64_t row, int64_t col, uint32_t rows) {
+    if (!aligned16(p)) return Load::kScalar;
+    if (col == 1 && row % 8 == 0 && g.k % 8 == 0) return Load::kK;
+    if (row == 1 && col % 8 == 0 && rows % 8 == 0) return Load::kOther;
+    return Load::kScalar;
+  };
+  const Load ma = mode(g.a, g.a_row, g.a_col, g.m), mb = mode(g.b, g.b_col, g.b_row, g.n);
   const dim3 grid(static_cast<uint32_t>(ceil_div(g.n, kBN)),
                   static_cast<uint32_t>(ceil_div(g.m, kBM)), splits);
-  if (af && bf)
-    hipLaunchKernelGGL((gemm_kernel<true, true>), grid, dim3(256), 0, st, a, kchunk);
-  else if (af)
-    hipLaunchKernelGGL((gemm_kernel<true, false>), grid, dim3(256), 0, st, a, kchunk);
-  else if (bf)
-    hipLaunchKernelGGL((gemm_kernel<false, true>), grid, dim3(256), 0, st, a, kchunk);
-  else
-    hipLaunchKernelGGL((gemm_kernel<false, false>), grid, dim3(256), 0, st, a, kchunk);
+  const auto with_mode = [](Load m, auto&& f) {
+    if (m == Load::kK) f(std::integral_constant<Load, Load::kK>{});
+    else if (m == Load::kOther) f(std::integral_constant<Load, Load::kOther>{});
+    else f(std::integral_constant<Load, Load::kScalar>{});
+  };
+  with_mode(ma, [&](auto x) {
+    with_mode(mb, [&](auto y) {
+      hipLaunchKernelGGL((gemm_kernel<decltype(x)::value, decltype(y)::value>), grid, dim3(256), 0,
+                         st, a, kchunk);
+    });
+  });
   launch_check("gemm_kernel");
   if (splits > 1) {
     const uint64_t mn = static_cast<uint64_t>(g.m) * g.n;
@@ -424,27 +463,45 @@ col2im_kernel(const float* __restrict__ dxcol, const uint16_t* __restrict__ ypre
   dy16[e] = to_bf16(g);
 }
 
-// Column sums of x [rows][cols] (FP32) in two passes: chunk partials, then
-// the chunks in order.
+// Column sums of x [rows][cols] (FP32) in two passes: a workgroup sums a chunk
+// of rows of 64 columns (four rows at a time, joined in LDS), then the chunks in
+// order.  Chunks are short (64 rows at 32576 rows of 64 columns) so that every CU
+// has some: chunks of 509 rows on one wave each took 97 us, these 5 us.
+constexpr uint32_t kColBlock = 64;  // columns per workgroup
+
 __global__ void __launch_bounds__(256)
-colsum_partial_kernel(const float* __restrict__ x, uint64_t rows, uint32_t cols,
+colsum_partial_kernel(const float* __restrict__ x, uint64_t rows, uint32_t cols, uint64_t per,
                       float* __restrict__ part) {
-  const uint32_t c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= cols) return;
-  const uint64_t per = ceil_div(rows, kColChunks);
+  __shared__ float red[4][kColBlock];
+  const uint32_t c = blockIdx.x * kColBlock + (threadIdx.x & 63u), group = threadIdx.x >> 6;
   const uint64_t r0 = blockIdx.y * per, r1 = min(rows, r0 + per);
   float s = 0.0f;
-  for (uint64_t r = r0; r < r1; ++r) s += x[r * cols + c];
-  part[static_cast<uint64_t>(blockIdx.y) * cols + c] = s;
+  if (c < cols) {
+#pragma unroll 8
+    for (uint64_t r = r0 + group; r < r1; r += 4) s += x[r * cols + c];
+  }
+  red[group][threadIdx.x & 63u] = s;
+  __syncthreads();
+  if (group == 0 && c < cols)
+    part[static_cast<uint64_t>(blockIdx.y) * cols + c] =
+        (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
 __global__ void __launch_bounds__(256)
-colsum_final_kernel(const float* __restrict__ part, uint32_t cols, float* __restrict__ out) {
-  const uint32_t c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= cols) return;
+colsum_final_kernel(const float* __restrict__ part, uint32_t cols, uint32_t chunks,
+                    float* __restrict__ out) {
+  __shared__ float red[4][kColBlock];
+  const uint32_t c = blockIdx.x * kColBlock + (threadIdx.x & 63u), group = threadIdx.x >> 6;
+  const uint32_t per = (chunks + 3) / 4, k1 = min(chunks, (group + 1) * per);
   float s = 0.0f;
-  for (uint32_t k = 0; k < kColChunks; ++k) s += part[static_cast<uint64_t>(k) * cols + c];
-  out[c] = s;
+  if (c < cols) {
+#pragma unroll 8
+    for (uint32_t k = group * per; k < k1; ++k) s += part[static_cast<uint64_t>(k) * cols + c];
+  }
+  red[group][threadIdx.x & 63u] = s;
+  __syncthreads();
+  if (group == 0 && c < cols)
+    out[c] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
 __global__ void __launch_bounds__(256)
@@ -515,11 +572,13 @@ dim3 blocks(uint64_t n) { return dim3(static_cast<uint32_t>(ceil_div(n, 256))); 
 
 void colsum(const float* x, uint64_t rows, uint32_t cols, float* part, float* out,
             hipStream_t st) {
-  hipLaunchKernelGGL(colsum_partial_kernel, dim3(static_cast<uint32_t>(ceil_div(cols, 256)),
-                                                 kColChunks),
-                     dim3(256), 0, st, x, rows, cols, part);
-  hipLaunchKernelGGL(colsum_final_kernel, dim3(static_cast<uint32_t>(ceil_div(cols, 256))),
-                     dim3(256), 0, st, part, cols, out);
+  const uint32_t most = kColChunks * kH / cols;  // what `part` holds
+  const uint64_t per = ceil_div(rows, std::max<uint64_t>(1, std::min<uint64_t>(most, rows / 64)));
+  const uint32_t chunks = static_cast<uint32_t>(ceil_div(rows, per));
+  const uint32_t cb = static_cast<uint32_t>(ceil_div(cols, kColBlock));
+  hipLaunchKernelGGL(colsum_partial_kernel, dim3(cb, chunks), dim3(256), 0, st, x, rows, cols, per,
+                     part);
+  hipLaunchKernelGGL(colsum_final_kernel, dim3(cb), dim3(256), 0, st, part, cols, chunks, out);
   launch_check("colsum_kernel");
 }
 
