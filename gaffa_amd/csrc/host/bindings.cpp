@@ -281,6 +281,7 @@ std::vector<std::pair<std::size_t, FfaPeak>> py_ffa_search_batch(
     GpuDeviceBuffer<float> d = upload(static_cast<const float*>(info.ptr), ns * n);
     GpuFfaExecutionOptions eo;
     eo.series_tile_size = series_tile;
+    eo.max_series = ns;
     GpuFfaProgram program(plan, GpuFfaProgramOptions{device_id}, eo);
     const FfaBatchSearchResult r = run_ffa_batch_gpu(
         program, GpuTimeSeriesBatchView{d.data(), ns, n, n, device_id},
@@ -615,6 +616,8 @@ PYBIND11_MODULE(_core, m) {
   m.attr("DM_PEAK_RECORD_BYTES") = sizeof(DmPeak);
   m.def("gpu_device_count", &gpu_device_count);
   m.def("gpu_runtime_version", &gpu_runtime_version);
+  m.def("release_device_cache", &release_device_cache,
+        "Give the device memory kept between calls back (at most 1/32 of each device's)");
   m.def("cuda_device_count", &gpu_device_count, "Alias of gpu_device_count for gaffa scripts.");
 
   py::register_exception_translator([](std::exception_ptr p) {

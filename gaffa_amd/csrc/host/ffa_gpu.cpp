@@ -346,6 +346,7 @@ GpuFfaProgram::GpuFfaProgram(const FfaSearchPlan& plan, const GpuFfaProgramOptio
   } else {
     tile_ = per_series == 0 ? 1024 : std::max<std::size_t>(1, exec_.workspace_bytes_limit / per_series);
     tile_ = std::min<std::size_t>(tile_, 1024);
+    if (exec_.max_series != 0) tile_ = std::min(tile_, exec_.max_series);
   }
   tile_ = std::min<std::size_t>(tile_, 65535);
   if (exec_.workspace_bytes_limit != 0 && exec_plan_.workspace_bytes(tile_) > exec_.workspace_bytes_limit &&
@@ -883,7 +884,9 @@ DmSearchResult find_dm_peaks_gpu(GpuDedispersedView<std::uint32_t> plane,
     hip_ok(gaffa_hip_detrend_normalise_batch(&a, nullptr), "convert_uint32_to_float");
     hip_ok(gaffa_hip_stream_synchronize(nullptr), "hipStreamSynchronize");
   }
-  GpuFfaProgram program(plan, GpuFfaProgramOptions{device_id});
+  GpuFfaExecutionOptions eo;
+  eo.max_series = plane.shape.ndm;
+  GpuFfaProgram program(plan, GpuFfaProgramOptions{device_id}, eo);
   const FfaSearchOptions fo{options.snr_threshold, options.max_peaks};
   GpuTimeSeriesBatchView batch{reinterpret_cast<const float*>(plane.data), plane.shape.ndm,
                                plane.shape.nsamples, stride, device_id};

@@ -25,6 +25,9 @@ struct GpuFfaExecutionOptions {
   // Series processed per launch sequence; 0 picks the largest tile whose
   // workspace fits workspace_bytes_limit.
   std::size_t series_tile_size = 0;
+  // Most series a run will have (0 = not known): a picked tile is no larger, so
+  // that a small batch does not allocate, and free, the limit's worth.
+  std::size_t max_series = 0;
   std::size_t workspace_bytes_limit = 16ULL << 30;
   std::size_t initial_peak_buffer_bytes = 64ULL << 20;
   std::size_t max_peak_buffer_bytes = 1ULL << 30;

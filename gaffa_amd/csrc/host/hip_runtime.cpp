@@ -2,10 +2,127 @@
 // status codes onto the exception classes gaffa throws.
 #include "gaffa/gpu_memory.h"
 
+#include <iterator>
+#include <list>
+#include <map>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 
 namespace gaffa {
+
+namespace {
+
+// Released device memory kept for reuse (see GpuDeviceMemory).  Every call is made
+// with the block's device current.
+class DeviceCache {
+ public:
+  // Never destroyed: the runtime may be gone before static destructors run.
+  static DeviceCache& get() {
+    static DeviceCache* cache = new DeviceCache;
+    return *cache;
+  }
+
+  // An allocation of at least `bytes`; `block` becomes its size.
+  void* take(int device, std::size_t bytes, std::size_t& block) {
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      auto best = blocks_.end();
+      for (auto it = blocks_.begin(); it != blocks_.end(); ++it)
+        if (it->device == device && it->bytes >= bytes && it->bytes - bytes <= bytes / 4 &&
+            (best == blocks_.end() || it->bytes < best->bytes))
+          best = it;
+      if (best != blocks_.end()) {
+        void* p = best->data;
+        block = best->bytes;
+        held_[device] -= block;
+        blocks_.erase(best);
+        return p;
+      }
+    }
+    void* p = nullptr;
+    block = bytes;
+    int status = gaffa_hip_malloc(&p, bytes);
+    if (status != GAFFA_HIP_OK && release(device)) status = gaffa_hip_malloc(&p, bytes);
+    hip_ok(status, "hipMalloc");
+    return p;
+  }
+
+  int give(int device, void* data, std::size_t bytes) {
+    if (bytes > limit(device)) return gaffa_hip_free(data);
+    // no kernel of any stream uses the block after this, as with hipFree
+    const int status = gaffa_hip_device_synchronize();
+    if (status != GAFFA_HIP_OK) {
+      (void)gaffa_hip_free(data);
+      return status;
+    }
+    std::list<Block> out;
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      blocks_.push_back(Block{device, data, bytes});
+      held_[device] += bytes;
+      for (auto it = blocks_.begin(); held_[device] > limit_[device];) {
+        const auto next = std::next(it);
+        if (it->device == device) {
+          held_[device] -= it->bytes;
+          out.splice(out.end(), blocks_, it);
+        }
+        it = next;
+      }
+    }
+    int freed = GAFFA_HIP_OK;
+    for (const Block& b : out) {
+      const int st = gaffa_hip_free(b.data);
+      if (freed == GAFFA_HIP_OK) freed = st;
+    }
+    return freed;
+  }
+
+  // Frees what is kept on `device`; whether there was anything.
+  bool release(int device) {
+    std::list<Block> out;
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      for (auto it = blocks_.begin(); it != blocks_.end();) {
+        const auto next = std::next(it);
+        if (it->device == device) out.splice(out.end(), blocks_, it);
+        it = next;
+      }
+      held_[device] = 0;
+    }
+    for (const Block& b : out) (void)gaffa_hip_free(b.data);
+    return !out.empty();
+  }
+
+ private:
+  struct Block {
+    int device;
+    void* data;
+    std::size_t bytes;
+  };
+
+  std::size_t limit(int device) {
+    std::lock_guard<std::mutex> lock(mutex_);
+    const auto it = limit_.find(device);
+    if (it != limit_.end()) return it->second;
+    gaffa_hip_device_info info{};
+    const bool ok = gaffa_hip_device_info_get(device, &info) == GAFFA_HIP_OK;
+    return limit_[device] = ok ? static_cast<std::size_t>(info.total_memory) / 32 : 0;
+  }
+
+  std::mutex mutex_;
+  std::list<Block> blocks_;  // oldest first
+  std::map<int, std::size_t> held_, limit_;
+};
+
+}  // namespace
+
+void release_device_cache() {
+  for (int d = 0; d < gpu_device_count(); ++d) {
+    GpuDeviceScope scope(d);
+    (void)DeviceCache::get().release(d);
+  }
+}
 
 void throw_hip_status(int status, const char* what) {
   const std::string msg = gaffa_hip_last_error();
@@ -41,7 +158,7 @@ GpuDeviceScope::~GpuDeviceScope() {
 GpuDeviceMemory::GpuDeviceMemory(std::size_t bytes) {
   int32_t dev = 0;
   hip_ok(gaffa_hip_get_device(&dev), "hipGetDevice");
-  if (bytes != 0) hip_ok(gaffa_hip_malloc(&data_, bytes), "hipMalloc");
+  if (bytes != 0) data_ = DeviceCache::get().take(dev, bytes, block_);
   bytes_ = bytes;
   device_id_ = dev;
 }
@@ -49,6 +166,7 @@ GpuDeviceMemory::GpuDeviceMemory(std::size_t bytes) {
 GpuDeviceMemory::GpuDeviceMemory(GpuDeviceMemory&& o) noexcept
     : data_(std::exchange(o.data_, nullptr)),
       bytes_(std::exchange(o.bytes_, 0)),
+      block_(std::exchange(o.block_, 0)),
       device_id_(std::exchange(o.device_id_, -1)) {}
 
 GpuDeviceMemory& GpuDeviceMemory::operator=(GpuDeviceMemory&& o) noexcept {
@@ -56,6 +174,7 @@ GpuDeviceMemory& GpuDeviceMemory::operator=(GpuDeviceMemory&& o) noexcept {
     release_noexcept();
     data_ = std::exchange(o.data_, nullptr);
     bytes_ = std::exchange(o.bytes_, 0);
+    block_ = std::exchange(o.block_, 0);
     device_id_ = std::exchange(o.device_id_, -1);
   }
   return *this;
@@ -66,10 +185,10 @@ GpuDeviceMemory::~GpuDeviceMemory() { release_noexcept(); }
 void GpuDeviceMemory::reset() {
   if (data_ != nullptr) {
     GpuDeviceScope scope(device_id_);
-    hip_ok(gaffa_hip_free(data_), "hipFree");
+    hip_ok(DeviceCache::get().give(device_id_, std::exchange(data_, nullptr), block_), "hipFree");
   }
-  data_ = nullptr;
   bytes_ = 0;
+  block_ = 0;
 }
 
 void GpuDeviceMemory::release_noexcept() noexcept {
@@ -77,10 +196,15 @@ void GpuDeviceMemory::release_noexcept() noexcept {
   int32_t cur = 0;
   const bool switch_dev = gaffa_hip_get_device(&cur) == 0 && cur != device_id_;
   if (switch_dev) (void)gaffa_hip_set_device(device_id_);
-  (void)gaffa_hip_free(data_);
+  try {
+    (void)DeviceCache::get().give(device_id_, data_, block_);
+  } catch (...) {  // no memory for the list's node
+    (void)gaffa_hip_free(data_);
+  }
   if (switch_dev) (void)gaffa_hip_set_device(cur);
   data_ = nullptr;
   bytes_ = 0;
+  block_ = 0;
 }
 
 GpuStream GpuStream::create() {

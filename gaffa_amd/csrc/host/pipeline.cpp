@@ -65,6 +65,7 @@ GpuSearchPipeline::GpuSearchPipeline(SearchPipelineConfig config) : cfg_(std::mo
   GpuFfaExecutionOptions fe;
   fe.workspace_bytes_limit = cfg_.ffa_workspace_bytes_limit;
   fe.series_tile_size = cfg_.ffa_series_tile;
+  fe.max_series = ndm_;
   fe.stream = stream_.get();
   // a full DM plane easily yields millions of significant peaks: start large
   // so the first run rarely repeats a tile

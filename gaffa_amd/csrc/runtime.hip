@@ -77,7 +77,10 @@ int gaffa_hip_malloc(void** ptr, uint64_t bytes) {
     check(ptr != nullptr, "allocation output must not be null");
     *ptr = nullptr;
     if (bytes == 0) return;
-    hip_check(hipMalloc(ptr, bytes), "hipMalloc");
+    const hipError_t err = hipMalloc(ptr, bytes);
+    // a caller may make room and try again: the next launch check must not see this
+    if (err != hipSuccess) (void)hipGetLastError();
+    hip_check(err, "hipMalloc");
   });
 }
 
