@@ -1494,6 +1494,38 @@ ffa_terminal_kernel(KArgs a, float* __restrict__ rows_out, uint32_t only_task) {
   }
 }
 
+// Merge table entries of a subtree node of `rows` rows (16 wave lists a pass).
+uint32_t subtree_entries(uint32_t rows) {
+  return subtree_tree_passes(tree_levels(rows)) * kSubtreeWaves * kSubtreeRowsPerPass *
+         subtree_passes(rows);
+}
+
+// Whether every node of the plan fits ffa_node_kernel.  Table sizes grow with
+// the rows, so the largest table bounds the rows of every node.
+bool nodes_in_registers(const gaffa_hip_ffa_plan_desc& p) {
+  return p.max_bins <= kNodeMaxBins && p.max_subtree_desc <= subtree_entries(kNodeMaxRows);
+}
+
+// Leaf rows of 8 level items a workgroup, a thread per row: stores bound it (36 MB
+// at 2^22 samples).  On the host, with the merge tables that plans in registers
+// never read, they were most of a one-shot search of one such series: 23 ms of
+// host work and upload, 3.6 ms in all with this.
+constexpr uint32_t kTableItems = 8;
+__global__ void __launch_bounds__(kTableItems * kLevelRowsMax)
+ffa_level_rows_kernel(const gaffa_hip_ffa_task* __restrict__ tasks,
+                      const gaffa_hip_ffa_item* __restrict__ items,
+                      const gaffa_hip_ffa_level_span* __restrict__ spans, uint32_t nitems,
+                      gaffa_hip_ffa_level_row* __restrict__ rows) {
+  const uint32_t k = blockIdx.x * kTableItems + threadIdx.x / kLevelRowsMax;
+  const uint32_t i = threadIdx.x % kLevelRowsMax;
+  if (k >= nitems) return;
+  const gaffa_hip_ffa_item it = items[k];
+  if (i >= it.c) return;
+  const gaffa_hip_ffa_task& t = tasks[it.task];
+  rows[spans[k].row_offset + i] =
+      level_leaves(t.rows, it.a & 0xFFFFu, it.a >> 16, it.b + i, t.bins);
+}
+
 void validate(const gaffa_hip_ffa_search_args* a) {
   check(a != nullptr && a->plan != nullptr, "FFA arguments must not be null");
   const gaffa_hip_ffa_plan_desc& p = *a->plan;
@@ -1518,7 +1550,7 @@ void validate(const gaffa_hip_ffa_search_args* a) {
   check(p.nsubtree_items == 0 ||
             (p.subtree_half_floats > 0 &&
              p.subtree_half_floats <= kSubtreePrefetch * kSubtreeThreads &&
-             (p.subtree_merges != nullptr || p.max_subtree_desc == 0) &&
+             (p.subtree_merges != nullptr || p.max_subtree_desc == 0 || nodes_in_registers(p)) &&
              8ull * p.subtree_half_floats + 4ull * kSubtreeGuard +
                      4ull * subtree_zero_floats(p.max_bins) <= p.subtree_lds_bytes),
         "FFA subtree geometry inconsistent");
@@ -1560,13 +1592,6 @@ int compute_units() {
     cus[dev] = n > 0 ? n : 1;
   }
   return cus[dev];
-}
-
-// Whether every node of the plan fits ffa_node_kernel.  Table sizes grow with
-// the rows, so the largest table bounds the rows of every node.
-bool nodes_in_registers(const gaffa_hip_ffa_plan_desc& p) {
-  static const uint32_t most = gaffa_hip_ffa_subtree_merges(kNodeMaxRows, 2, nullptr);
-  return p.max_bins <= kNodeMaxBins && p.max_subtree_desc <= most;
 }
 
 void launch_prepare(const gaffa_hip_ffa_search_args* a, hipStream_t st) {
@@ -1731,6 +1756,27 @@ int gaffa_hip_ffa_reserve_launch(const gaffa_hip_ffa_plan_desc* p) {
   });
 }
 
+int gaffa_hip_ffa_build_level_rows(const gaffa_hip_ffa_task* tasks,
+                                   const gaffa_hip_ffa_item* items,
+                                   const gaffa_hip_ffa_level_span* spans, uint32_t nitems,
+                                   gaffa_hip_ffa_level_row* rows, gaffa_hip_stream stream) {
+  return guarded([&] {
+    check(nitems == 0 || (tasks != nullptr && items != nullptr && spans != nullptr &&
+                          rows != nullptr),
+          "FFA level tables must not be null");
+    if (nitems == 0) return;
+    hipLaunchKernelGGL(ffa_level_rows_kernel,
+                       dim3(static_cast<uint32_t>(ceil_div(nitems, kTableItems))),
+                       dim3(kTableItems * kLevelRowsMax), 0, as_stream(stream), tasks, items, spans,
+                       nitems, rows);
+    launch_check("ffa_level_rows_kernel");
+  });
+}
+
+uint32_t gaffa_hip_ffa_subtree_reads_merges(uint32_t max_rows, uint32_t max_bins) {
+  return max_rows > kNodeMaxRows || max_bins > kNodeMaxBins ? 1u : 0u;
+}
+
 uint32_t gaffa_hip_ffa_prepare_outputs_per_block(double factor) {
   return prep_outputs_per_block(factor);
 }
@@ -1748,7 +1794,12 @@ uint64_t gaffa_hip_ffa_level_item(uint32_t task_rows, uint32_t bins, uint32_t de
     return ~uint64_t{0};
   const uint32_t nleaf = 1u << levels;
   uint32_t lo[8] = {}, hi[8] = {};
-  for (uint32_t i = 0; i < count; ++i) {
+  // inside one node every leaf is monotone in the row: the first and last rows
+  // have its runs
+  const bool one_node = find_node(0, task_rows, depth, first).start ==
+                        find_node(0, task_rows, depth, first + count - 1).start;
+  const uint32_t step = rows == nullptr && one_node && count > 1 ? count - 1 : 1;
+  for (uint32_t i = 0; i < count; i += step) {
     const gaffa_hip_ffa_level_row e = level_leaves(task_rows, depth, levels, first + i, bins);
     if (rows != nullptr) rows[i] = e;
     for (uint32_t j = 0; j < nleaf; ++j) {

@@ -126,7 +126,8 @@ void GpuFfaBatchedSearch::build_tiles() {
     t->merges = gaffa::upload(e.subtree_merges().data(), e.subtree_merges().size());
     t->level = gaffa::upload(e.level_items().data(), e.level_items().size());
     t->level_spans = gaffa::upload(e.level_spans().data(), e.level_spans().size());
-    t->level_rows = gaffa::upload(e.level_leaf_rows().data(), e.level_leaf_rows().size());
+    t->level_rows = e.build_level_leaf_rows(t->tasks.data(), t->level.data(),
+                                            t->level_spans.data(), stream_.get());
     t->terminal = gaffa::upload(e.terminal_items().data(), e.terminal_items().size());
     gaffa_hip_ffa_plan_desc& d = t->desc;
     d.groups = t->groups.data();

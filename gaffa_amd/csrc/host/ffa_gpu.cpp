@@ -111,8 +111,66 @@ GpuFfaExecutionPlan::GpuFfaExecutionPlan(const FfaSearchPlan& plan, FfaItemShape
   input_nsamples_ = plan.tasks.front().input_nsamples;
   check_arg(input_nsamples_ > 0, "FFA executor time series must not be empty");
   lds_max_bins_ = plan_max_bins(plan);
+  const FfaSearchPlan* const one = &plan;
+  find_needs_merges({&one, 1});
   append(plan, 0, 0);
   finish();
+}
+
+std::size_t GpuFfaExecutionPlan::lds_rows(std::size_t bins) const {
+  check_arg(subtree_fixed_lds(lds_max_bins_) < kSubtreeLdsBytes,
+            "GPU FFA bins too large for an LDS subtree");
+  // two ping-pong buffers in what the fixed LDS leaves
+  const std::size_t node_floats = (kSubtreeLdsBytes - subtree_fixed_lds(lds_max_bins_)) / 8;
+  const std::size_t rows = std::min(kSubtreeMaxRows, node_floats / bins);
+  check_arg(rows >= 2, "GPU FFA bins too large for an LDS subtree");
+  return rows;
+}
+
+std::uint32_t GpuFfaExecutionPlan::lds_depth(std::size_t rows, std::size_t bins) const {
+  const std::size_t fit = lds_rows(bins);
+  std::uint32_t depth = 1;
+  while ((rows + (std::size_t{1} << depth) - 1) >> depth > fit) ++depth;
+  return depth;
+}
+
+// Whether some node is beyond the kernel that reads no merge tables; tasks that
+// append() refuses do not matter here.
+void GpuFfaExecutionPlan::find_needs_merges(std::span<const FfaSearchPlan* const> plans) {
+  if (subtree_fixed_lds(lds_max_bins_) >= kSubtreeLdsBytes) return;
+  const std::size_t node_floats = (kSubtreeLdsBytes - subtree_fixed_lds(lds_max_bins_)) / 8;
+  std::size_t most = 0;
+  for (const FfaSearchPlan* plan : plans)
+    for (const FfaSearchTask& t : plan->tasks) {
+      if (t.rows < 2 || t.bins < 2 || t.rows >= (std::size_t{1} << 31) || node_floats / t.bins < 2)
+        continue;
+      const std::uint32_t depth = lds_depth(t.rows, t.bins);
+      most = std::max(most, (t.rows + (std::size_t{1} << depth) - 1) >> depth);
+    }
+  needs_merges_ = gaffa_hip_ffa_subtree_reads_merges(static_cast<std::uint32_t>(most),
+                                                     static_cast<std::uint32_t>(lds_max_bins_)) != 0;
+}
+
+GpuDeviceBuffer<gaffa_hip_ffa_level_row> GpuFfaExecutionPlan::build_level_leaf_rows(
+    const gaffa_hip_ffa_task* tasks, const gaffa_hip_ffa_item* items,
+    const gaffa_hip_ffa_level_span* spans, gaffa_hip_stream stream) const {
+  GpuDeviceBuffer<gaffa_hip_ffa_level_row> rows(level_row_count_);
+  hip_ok(gaffa_hip_ffa_build_level_rows(tasks, items, spans,
+                                        static_cast<std::uint32_t>(level_.size()), rows.data(),
+                                        stream),
+         "ffa_build_level_rows");
+  return rows;
+}
+
+std::vector<gaffa_hip_ffa_level_row> GpuFfaExecutionPlan::level_leaf_rows() const {
+  std::vector<gaffa_hip_ffa_level_row> rows(level_row_count_);
+  for (std::size_t k = 0; k < level_.size(); ++k) {
+    const gaffa_hip_ffa_item& it = level_[k];
+    const gaffa_hip_ffa_task& t = tasks_[it.task];
+    (void)gaffa_hip_ffa_level_item(t.rows, t.bins, it.a & 0xFFFFu, it.a >> 16, it.b, it.c, nullptr,
+                                   rows.data() + level_spans_[k].row_offset);
+  }
+  return rows;
 }
 
 GpuFfaExecutionPlan::GpuFfaExecutionPlan(std::span<const FfaBatchMember> members,
@@ -124,8 +182,13 @@ GpuFfaExecutionPlan::GpuFfaExecutionPlan(std::span<const FfaBatchMember> members
                              "FFA terminal rows per item too large");
   check_arg(!members.empty(), "FFA batch must contain at least one series");
   plan_.width_trials = members.front().plan->width_trials;
+  std::vector<const FfaSearchPlan*> plans;
   for (const FfaBatchMember& m : members)
-    if (m.plan != nullptr) lds_max_bins_ = std::max(lds_max_bins_, plan_max_bins(*m.plan));
+    if (m.plan != nullptr) {
+      lds_max_bins_ = std::max(lds_max_bins_, plan_max_bins(*m.plan));
+      plans.push_back(m.plan);
+    }
+  find_needs_merges(plans);
   for (const FfaBatchMember& m : members) {
     check_arg(m.plan != nullptr && !m.plan->tasks.empty(),
               "FFA executor plan must contain at least one task");
@@ -200,16 +263,10 @@ void GpuFfaExecutionPlan::append(const FfaSearchPlan& plan, std::uint64_t input_
         terminal_lds_bytes_,
         gaffa_hip_ffa_terminal_lds_bytes_rows(d.bins, static_cast<std::uint32_t>(det.max_width),
                                               terminal_rows));
-    // rows of a node: two ping-pong buffers in what the fixed LDS leaves
-    check_arg(subtree_fixed_lds(lds_max_bins_) < kSubtreeLdsBytes,
-              "GPU FFA bins too large for an LDS subtree");
-    const std::size_t node_floats = (kSubtreeLdsBytes - subtree_fixed_lds(lds_max_bins_)) / 8;
-    const std::size_t lds_rows = std::min(kSubtreeMaxRows, node_floats / t.bins);
-    check_arg(lds_rows >= 2, "GPU FFA bins too large for an LDS subtree");
+    (void)lds_rows(t.bins);  // refuses bins too large for an LDS subtree
     const std::uint32_t task_index = static_cast<std::uint32_t>(tasks_.size());
     if (t.rows >= 2) {
-      std::uint32_t depth = 1;
-      while ((t.rows + (std::size_t{1} << depth) - 1) >> depth > lds_rows) ++depth;
+      const std::uint32_t depth = lds_depth(t.rows, t.bins);
       d.depth = depth;
       d.work_offset = work_stride_;
       work_stride_ += align_up(t.rows * t.bins);
@@ -223,6 +280,7 @@ void GpuFfaExecutionPlan::append(const FfaSearchPlan& plan, std::uint64_t input_
         const std::uint32_t entries = gaffa_hip_ffa_subtree_merges(it.b, d.bins, nullptr);
         check_arg(entries > 0 || it.b < 2, "GPU FFA subtree merge table unavailable");
         subtree_desc_ = std::max(subtree_desc_, entries);
+        if (!needs_merges_) continue;
         // one merge table per (rows, bins), shared by every node of that shape
         auto [pos, fresh] = merge_table_of_.try_emplace(
             (std::uint64_t{it.b} << 32) | d.bins, static_cast<std::uint32_t>(merges_.size()));
@@ -278,13 +336,12 @@ void GpuFfaExecutionPlan::append(const FfaSearchPlan& plan, std::uint64_t input_
             by_depth_[dout].push_back(
                 gaffa_hip_ffa_item{task_index, dout | (levels << 16), r, count});
             gaffa_hip_ffa_level_span span{};
-            check_arg(level_leaf_rows_.size() + count < (std::size_t{1} << 32),
+            check_arg(level_row_count_ + count < (std::size_t{1} << 32),
                       "FFA plan has too many level rows");
-            span.row_offset = static_cast<std::uint32_t>(level_leaf_rows_.size());
-            level_leaf_rows_.resize(level_leaf_rows_.size() + count);
-            const std::uint64_t need = gaffa_hip_ffa_level_item(
-                d.rows, d.bins, dout, levels, r, count, &span,
-                level_leaf_rows_.data() + span.row_offset);
+            span.row_offset = static_cast<std::uint32_t>(level_row_count_);
+            level_row_count_ += count;
+            const std::uint64_t need = gaffa_hip_ffa_level_item(d.rows, d.bins, dout, levels, r,
+                                                                count, &span, nullptr);
             check_arg(need != ~std::uint64_t{0}, "FFA level item outside its task");
             spans_by_depth_[dout].push_back(span);
             if (need <= kLevelLdsCap)
@@ -361,7 +418,8 @@ GpuFfaProgram::GpuFfaProgram(const FfaSearchPlan& plan, const GpuFfaProgramOptio
   d_merges_ = upload(exec_plan_.subtree_merges().data(), exec_plan_.subtree_merges().size());
   d_level_ = upload(exec_plan_.level_items().data(), exec_plan_.level_items().size());
   d_level_spans_ = upload(exec_plan_.level_spans().data(), exec_plan_.level_spans().size());
-  d_level_rows_ = upload(exec_plan_.level_leaf_rows().data(), exec_plan_.level_leaf_rows().size());
+  d_level_rows_ = exec_plan_.build_level_leaf_rows(d_tasks_.data(), d_level_.data(),
+                                                   d_level_spans_.data(), exec_.stream);
   d_terminal_ = upload(exec_plan_.terminal_items().data(), exec_plan_.terminal_items().size());
   prepared_ = GpuDeviceBuffer<float>(std::max<std::size_t>(1, tile_ * exec_plan_.prepared_stride()));
   work_ = GpuDeviceBuffer<float>(std::max<std::size_t>(1, 2 * tile_ * exec_plan_.work_stride()));

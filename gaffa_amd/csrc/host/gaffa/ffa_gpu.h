@@ -90,9 +90,13 @@ class GpuFfaExecutionPlan {
   const std::vector<gaffa_hip_ffa_merge>& subtree_merges() const noexcept { return merges_; }
   const std::vector<gaffa_hip_ffa_item>& level_items() const noexcept { return level_; }
   const std::vector<gaffa_hip_ffa_level_span>& level_spans() const noexcept { return level_spans_; }
-  const std::vector<gaffa_hip_ffa_level_row>& level_leaf_rows() const noexcept {
-    return level_leaf_rows_;
-  }
+  // Leaf rows of all level items (the spans' row_offset): built on the device
+  // from the uploaded tasks, items and spans, enqueued on `stream`.
+  GpuDeviceBuffer<gaffa_hip_ffa_level_row> build_level_leaf_rows(
+      const gaffa_hip_ffa_task* tasks, const gaffa_hip_ffa_item* items,
+      const gaffa_hip_ffa_level_span* spans, gaffa_hip_stream stream) const;
+  // The same rows on the host.
+  std::vector<gaffa_hip_ffa_level_row> level_leaf_rows() const;
   const std::vector<std::uint32_t>& level_offsets() const noexcept { return level_offsets_; }
   const std::vector<gaffa_hip_ffa_item>& terminal_items() const noexcept { return terminal_; }
   std::uint32_t subtree_lds_bytes() const noexcept { return subtree_lds_bytes_; }
@@ -115,7 +119,7 @@ class GpuFfaExecutionPlan {
   std::vector<std::vector<gaffa_hip_ffa_item>> by_depth_;
   std::vector<std::vector<gaffa_hip_ffa_level_span>> spans_by_depth_;
   std::vector<gaffa_hip_ffa_level_span> level_spans_;   // parallel to level_
-  std::vector<gaffa_hip_ffa_level_row> level_leaf_rows_;
+  std::size_t level_row_count_ = 0;
   FfaSearchPlan plan_;
   std::size_t input_nsamples_ = 0;
   std::size_t prepared_stride_ = 0;
@@ -123,6 +127,11 @@ class GpuFfaExecutionPlan {
   std::size_t max_depth_ = 0;
   std::size_t max_prepared_ = 0;
   std::size_t lds_max_bins_ = 0;  // bins of the widest task of every plan appended
+  bool needs_merges_ = true;      // the subtree kernel reads the merge tables
+  // rows of a subtree node in LDS, and the depth of the first nodes that fit
+  std::size_t lds_rows(std::size_t bins) const;
+  std::uint32_t lds_depth(std::size_t rows, std::size_t bins) const;
+  void find_needs_merges(std::span<const FfaSearchPlan* const> plans);
   std::uint32_t level_rows_ = 0, terminal_rows_ = 0;  // rows per level / terminal item
   std::uint32_t subtree_lds_bytes_ = 0;
   std::uint32_t subtree_half_ = 0;

@@ -420,7 +420,8 @@ typedef struct gaffa_hip_ffa_plan_desc {
   uint32_t ntasks;
   const gaffa_hip_ffa_item* subtree_items; /* device; c = first merge */
   uint32_t nsubtree_items;
-  const gaffa_hip_ffa_merge* subtree_merges; /* device */
+  const gaffa_hip_ffa_merge* subtree_merges; /* device; may be null where
+                                  ..._subtree_reads_merges() says 0 */
   const gaffa_hip_ffa_item* level_items;   /* device, sorted by depth desc */
   const gaffa_hip_ffa_level_span* level_spans;    /* device, one per level item */
   const gaffa_hip_ffa_level_row* level_leaf_rows; /* device, spans' row tables */
@@ -486,7 +487,18 @@ uint64_t gaffa_hip_ffa_level_lds_bytes(uint32_t task_rows, uint32_t bins, uint32
 uint64_t gaffa_hip_ffa_level_item(uint32_t task_rows, uint32_t bins, uint32_t depth,
                                   uint32_t levels, uint32_t first, uint32_t count,
                                   gaffa_hip_ffa_level_span* span, gaffa_hip_ffa_level_row* rows);
+/* The leaf rows of `nitems` level items on the device, as
+ * gaffa_hip_ffa_level_item gives them: rows[spans[k].row_offset + i] for row i
+ * of item k (all pointers device; tasks as in the plan).  No gaffa counterpart. */
+int gaffa_hip_ffa_build_level_rows(const gaffa_hip_ffa_task* tasks,
+                                   const gaffa_hip_ffa_item* items,
+                                   const gaffa_hip_ffa_level_span* spans, uint32_t nitems,
+                                   gaffa_hip_ffa_level_row* rows, gaffa_hip_stream stream);
 uint32_t gaffa_hip_ffa_subtree_lds_bytes(uint32_t rows, uint32_t bins);
+/* 1 if the subtree launch of a plan whose nodes hold at most `max_rows` rows of
+ * at most `max_bins` bins reads the merge tables; else subtree_merges may be null
+ * (max_subtree_desc is the tables' size all the same). */
+uint32_t gaffa_hip_ffa_subtree_reads_merges(uint32_t max_rows, uint32_t max_bins);
 /* Fills the merge table of a subtree node of `rows` rows (host memory; a
  * null `out` only counts) with the kernels' own row-selection arithmetic
  * (gaffa's ffa.cpp:133-143 in FP32).  Returns the entry count, 0 for rows

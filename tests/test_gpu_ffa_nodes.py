@@ -32,3 +32,45 @@ def test_ffa_nodes_bit_exact(gpu, port, bins):
         for k in range(3):
             want = port.ffa_transform(x[k, : rows * bins], bins)
             np.testing.assert_array_equal(got[k], want)
+
+
+@pytest.mark.parametrize("nsamples,level_rows", [(1 << 20, 0), (1 << 21, 7), (1 << 18, 0)])
+def test_level_rows_built_on_the_device(gpu, nsamples, level_rows):
+    """The leaf rows the device builds for a plan's level items (whole items,
+    short ones, a last workgroup that is not full, a plan with none) are the
+    host's, entry for entry."""
+    import ctypes
+
+    import gaffa_amd
+    from gaffa_amd.ffa import make_riptide_plan
+
+    plan = make_riptide_plan(nsamples=nsamples, tsamp=6.4e-5, period_min=0.1, period_max=10.0,
+                             duty_cycle_max=0.18, width_trial_spacing=2.0)
+    d = gpu._ffa_level_layout(plan, level_rows)
+    items, spans, want = (np.ascontiguousarray(d[k]) for k in ("items", "spans", "leaf_rows"))
+    print(f"level rows: {len(items)} items, {len(want)} rows", flush=True)
+    tasks = np.zeros((plan.task_count, 62), np.uint32)  # gaffa_hip_ffa_task: bins, rows
+    tasks[:, 1], tasks[:, 2] = plan.tasks["bins"], plan.tasks["rows"]
+    lib = ctypes.CDLL(gaffa_amd.HIP_LIBRARY)
+    ptrs = []
+
+    def put(arr):
+        p = ctypes.c_void_p()
+        assert lib.gaffa_hip_malloc(ctypes.byref(p), ctypes.c_uint64(max(arr.nbytes, 256))) == 0
+        ptrs.append(p)
+        assert lib.gaffa_hip_memcpy(p, arr.ctypes.data_as(ctypes.c_void_p),
+                                    ctypes.c_uint64(arr.nbytes), None) == 0
+        return p
+
+    try:
+        out = np.full(want.shape, 0xABABABAB, np.uint32)
+        args = [put(tasks), put(items), put(spans)]
+        dev = put(out)
+        assert lib.gaffa_hip_ffa_build_level_rows(*args, ctypes.c_uint32(len(items)), dev,
+                                                  None) == 0
+        assert lib.gaffa_hip_memcpy(out.ctypes.data_as(ctypes.c_void_p), dev,
+                                    ctypes.c_uint64(out.nbytes), None) == 0
+    finally:
+        for p in ptrs:
+            lib.gaffa_hip_free(p)
+    np.testing.assert_array_equal(out, want)
