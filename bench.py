@@ -85,7 +85,7 @@ KERNEL_NAMES = {
     "dedisperse": "dedisperse_subband_stream_kernel",
     "ffa": "FFA stage (prepare + subtree + levels + detect)",
     "ffa_prepare": "ffa_prepare_fused_kernel",
-    "ffa_subtree": "ffa_subtree_kernel",
+    "ffa_subtree": "ffa_node_kernel",
     "ffa_levels": "ffa_level_kernel",
     "ffa_detect": "ffa_terminal_kernel<true>",
 }

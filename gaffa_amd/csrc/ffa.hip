@@ -28,9 +28,10 @@
 //             P[phi + w], so every boxcar sum equals the CPU's circular-prefix
 //             difference bit for bit (ffa_detection.cpp:126-239); significant
 //             peaks are appended with one atomic each.
-// The LDS subtree and level kernels read their merges and leaves from
-// host-built tables; in the terminal kernel the (head row, tail row, roll) descriptor of
-// each output row is computed once, by one lane, into LDS.  The waves then
+// The LDS subtree and level kernels read their merges and leaves from the
+// plan's tables (the leaves built on the device); in the terminal kernel the
+// (head row, tail row, roll) descriptor of each output row is computed once, by
+// one lane, into LDS.  The waves then
 // stream whole rows (lanes over phase bins) reading only those.  The subtree
 // and level passes write their rows with streaming stores.
 #include "common.hpp"
@@ -226,7 +227,7 @@ __device__ __host__ __forceinline__ uint32_t prep_outputs_per_block(double facto
 // w0 src[first] + src[first + 1] + ... + src[last - 1] + w1 src[last], added in
 // that order: one chain of adds an output, so eight samples are read ahead of
 // their adds: a read per add waits for LDS each time.  In the kernel of one
-// group: 200 us a launch before, 78 us now (octaves of 64 series, 6 launches).
+// group: 200 us a launch before, 78 us now (octaves of 96 series, 6 launches).
 template <typename S, typename I>
 __device__ __forceinline__ float weighted_sum(S src, I first, I last, float w0, float w1) {
   float sum = w0 * src[first];
@@ -294,7 +295,7 @@ ffa_prepare_kernel(const float* __restrict__ series, uint64_t series_stride,
 // group.  The chains of adds of the largest factors bound it (a few outputs a
 // span, hundreds of adds each), hence their place at the front and the reads
 // ahead: 1168 us a launch with a read per add and the longest last, 587 us now
-// (lband search, 256 DM series of 262144 samples).
+// (lband search, 256 DM series of 2^20 samples).
 constexpr uint32_t kPrepSpan = 8192;
 constexpr uint32_t kPrepMaxHalo = 4096;
 constexpr uint32_t kPrepMaxGroups = 64;
@@ -1147,7 +1148,7 @@ __host__ __device__ __forceinline__ uint64_t level_stage_bytes(uint32_t staged_r
 // Rows [item.b, item.b + item.c) of the depth-d nodes of a task (item.a = d
 // | L << 16).  The item's leaf runs (its span, host-built) are copied into
 // LDS once (global_load_lds: 64 consecutive floats per instruction, straight
-// into LDS) together with its rows' leaves (host-built), and each output
+// into LDS) together with its rows' leaves (the plan's), and each output
 // phase then reads its 2^L operands there; a wave merges one row at a time,
 // four 64-phase chunks per block.  An item whose runs exceed the launch's LDS
 // (plan.level_lds_bytes) reads its operands from global memory instead, with
