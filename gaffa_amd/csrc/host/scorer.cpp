@@ -86,6 +86,10 @@ void GpuCandidateScorer::set_parameters(std::span<const float> values) {
   GpuDeviceScope scope(device_id_);
   const gaffa_hip_scorer_net n = net();
   copy_to_device(params_.data(), values.data(), nparams_ * sizeof(float), stream_.get());
+  // the gradients too: no layer writes the padding of the parameter vector
+  hip_ok(gaffa_hip_fill_u32(reinterpret_cast<std::uint32_t*>(grads_.data()), 0, nparams_,
+                            stream_.get()),
+         "fill_u32");
   hip_ok(gaffa_hip_fill_u32(reinterpret_cast<std::uint32_t*>(adam_m_.data()), 0, nparams_,
                             stream_.get()),
          "fill_u32");

@@ -44,3 +44,34 @@ def test_reused_device_memory_keeps_results(gpu):
     gpu.release_device_cache()
     work([2, 1, 0])
     assert bad == []
+
+
+def test_gradient_padding_is_zero_in_used_memory(gpu):
+    """The parameter vector is padded to a multiple of 8; its gradient there is
+    zero, also where the scorer's buffers held another call's data before."""
+    import gaffa_amd
+    from oracle import scorer_oracle as so
+
+    gpu.release_device_cache()
+    size = gaffa_amd.CandidateScorer(capacity=8).parameters.size
+    rng = np.random.default_rng(6)
+    x = rng.integers(1, 4000, size=(1, size + size // 8)).astype(np.uint32)
+
+    def leave():
+        for _ in range(4):
+            gpu._preprocess_batch_gpu(x, window_samples=None, normalise=True)
+
+    threads = [threading.Thread(target=leave) for _ in range(6)]
+    gpu.release_device_cache()
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    s = gaffa_amd.CandidateScorer(capacity=8)
+    _, g = s.gradients(rng.normal(size=(8, so.SUBINTS, so.PHASE)).astype(np.float32),
+                       rng.normal(size=(8, so.PATCH)).astype(np.float32),
+                       np.ones(8, np.float32))
+    lay = so.layout()
+    used = lay["bias"][5] + 1
+    assert g.size == size and used < size
+    np.testing.assert_array_equal(g[used:], 0.0)
