@@ -51,9 +51,9 @@ class GpuDeviceScope {
 // the oldest goes back first, and all of it when an allocation would fail or on
 // release_device_cache().  hipMalloc of memory that was used before costs about
 // 24 ms a GB (the driver clears it): a one-shot search of 24 series of 524291
-// samples, 3 GB of workspace, spent 74 of its 85 ms there.  The device is
-// synchronised before a block is kept, as hipFree does, so whatever stream used
-// it is done; a block's contents are not cleared.
+// samples, 3 GB of workspace, spent 74 of its 85 ms there.  The release waits for
+// the device before a block is kept, as hipFree does, so whatever stream used it
+// is done; a block's contents are not cleared.
 class GpuDeviceMemory {
  public:
   GpuDeviceMemory() = default;

@@ -51,7 +51,7 @@ class DeviceCache {
   int give(int device, void* data, std::size_t bytes) {
     if (bytes > limit(device)) return gaffa_hip_free(data);
     // no kernel of any stream uses the block after this, as with hipFree
-    const int status = gaffa_hip_device_synchronize();
+    const int status = wait_for_device();
     if (status != GAFFA_HIP_OK) {
       (void)gaffa_hip_free(data);
       return status;
@@ -100,6 +100,16 @@ class DeviceCache {
     void* data;
     std::size_t bytes;
   };
+
+  // Waits until the device is idle by freeing an allocation of a byte (under 1 us
+  // on an idle device): hipFree waits as hipDeviceSynchronize does, but a device
+  // synchronisation is refused while another thread captures a graph, and ends
+  // that capture with an error.
+  static int wait_for_device() {
+    void* token = nullptr;
+    const int status = gaffa_hip_malloc(&token, 1);
+    return status == GAFFA_HIP_OK ? gaffa_hip_free(token) : status;
+  }
 
   std::size_t limit(int device) {
     std::lock_guard<std::mutex> lock(mutex_);

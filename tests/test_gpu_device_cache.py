@@ -75,3 +75,39 @@ def test_gradient_padding_is_zero_in_used_memory(gpu):
     used = lay["bias"][5] + 1
     assert g.size == size and used < size
     np.testing.assert_array_equal(g[used:], 0.0)
+
+
+def test_release_beside_a_capture(gpu):
+    """Device memory released by one thread leaves a graph that another thread
+    captures (thread-local mode) whole: it ends, and every replay writes."""
+    import ctypes
+
+    import gaffa_amd
+
+    lib = ctypes.CDLL(gaffa_amd.HIP_LIBRARY)
+    stream, graph, out = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    words = 1024
+    held = [gaffa_amd.CandidateScorer(capacity=8)]
+    assert lib.gaffa_hip_stream_create(ctypes.byref(stream)) == 0
+    assert lib.gaffa_hip_malloc(ctypes.byref(out), ctypes.c_uint64(4 * words)) == 0
+    try:
+        assert lib.gaffa_hip_graph_begin(stream) == 0
+        queued = lib.gaffa_hip_fill_u32(out, 7, ctypes.c_uint64(words), stream)
+        worker = threading.Thread(target=held.clear)  # the last reference
+        worker.start()
+        worker.join()
+        ended = lib.gaffa_hip_graph_end(stream, ctypes.byref(graph))
+        assert held == [] and (queued, ended) == (0, 0)
+        got = np.empty(words, np.uint32)
+        for _ in range(3):
+            assert lib.gaffa_hip_memset(out, 0, ctypes.c_uint64(4 * words), None) == 0
+            assert lib.gaffa_hip_graph_launch(graph, stream) == 0
+            assert lib.gaffa_hip_stream_synchronize(stream) == 0
+            assert lib.gaffa_hip_memcpy(got.ctypes.data_as(ctypes.c_void_p), out,
+                                        ctypes.c_uint64(4 * words), None) == 0
+            assert (got == 7).all()
+    finally:
+        if graph.value:
+            lib.gaffa_hip_graph_destroy(graph)
+        lib.gaffa_hip_stream_destroy(stream)
+        lib.gaffa_hip_free(out)
