@@ -35,7 +35,7 @@ class DeviceCache {
       if (best != blocks_.end()) {
         void* p = best->data;
         block = best->bytes;
-        held_[device] -= block;
+        devices_.find(device)->second.bytes -= block;
         blocks_.erase(best);
         return p;
       }
@@ -48,23 +48,30 @@ class DeviceCache {
     return p;
   }
 
-  int give(int device, void* data, std::size_t bytes) {
-    if (bytes > limit(device)) return gaffa_hip_free(data);
+  int give(int device, void* data, std::size_t bytes) noexcept {
+    std::list<Block> own, out;
+    Device* held = nullptr;
+    try {  // all that can fail for want of host memory comes before the block is listed
+      own.push_back(Block{device, data, bytes});
+      held = &state(device);
+    } catch (...) {
+      return gaffa_hip_free(data);
+    }
+    if (bytes > held->limit) return gaffa_hip_free(data);
     // no kernel of any stream uses the block after this, as with hipFree
     const int status = wait_for_device();
     if (status != GAFFA_HIP_OK) {
       (void)gaffa_hip_free(data);
       return status;
     }
-    std::list<Block> out;
     {
       std::lock_guard<std::mutex> lock(mutex_);
-      blocks_.push_back(Block{device, data, bytes});
-      held_[device] += bytes;
-      for (auto it = blocks_.begin(); held_[device] > limit_[device];) {
+      blocks_.splice(blocks_.end(), own);
+      held->bytes += bytes;
+      for (auto it = blocks_.begin(); held->bytes > held->limit;) {
         const auto next = std::next(it);
         if (it->device == device) {
-          held_[device] -= it->bytes;
+          held->bytes -= it->bytes;
           out.splice(out.end(), blocks_, it);
         }
         it = next;
@@ -85,10 +92,12 @@ class DeviceCache {
       std::lock_guard<std::mutex> lock(mutex_);
       for (auto it = blocks_.begin(); it != blocks_.end();) {
         const auto next = std::next(it);
-        if (it->device == device) out.splice(out.end(), blocks_, it);
+        if (it->device == device) {
+          devices_.find(device)->second.bytes -= it->bytes;
+          out.splice(out.end(), blocks_, it);
+        }
         it = next;
       }
-      held_[device] = 0;
     }
     for (const Block& b : out) (void)gaffa_hip_free(b.data);
     return !out.empty();
@@ -99,6 +108,10 @@ class DeviceCache {
     int device;
     void* data;
     std::size_t bytes;
+  };
+  struct Device {
+    std::size_t bytes = 0;  // kept
+    std::size_t limit = 0;
   };
 
   // Waits until the device is idle by freeing an allocation of a byte (under 1 us
@@ -111,18 +124,21 @@ class DeviceCache {
     return status == GAFFA_HIP_OK ? gaffa_hip_free(token) : status;
   }
 
-  std::size_t limit(int device) {
+  // A device's entry, made at its first release (a map's entries never move).
+  Device& state(int device) {
     std::lock_guard<std::mutex> lock(mutex_);
-    const auto it = limit_.find(device);
-    if (it != limit_.end()) return it->second;
-    gaffa_hip_device_info info{};
-    const bool ok = gaffa_hip_device_info_get(device, &info) == GAFFA_HIP_OK;
-    return limit_[device] = ok ? static_cast<std::size_t>(info.total_memory) / 32 : 0;
+    const auto [it, fresh] = devices_.try_emplace(device);
+    if (fresh) {
+      gaffa_hip_device_info info{};
+      const bool ok = gaffa_hip_device_info_get(device, &info) == GAFFA_HIP_OK;
+      it->second.limit = ok ? static_cast<std::size_t>(info.total_memory) / 32 : 0;
+    }
+    return it->second;
   }
 
   std::mutex mutex_;
   std::list<Block> blocks_;  // oldest first
-  std::map<int, std::size_t> held_, limit_;
+  std::map<int, Device> devices_;
 };
 
 }  // namespace
@@ -195,10 +211,12 @@ GpuDeviceMemory::~GpuDeviceMemory() { release_noexcept(); }
 void GpuDeviceMemory::reset() {
   if (data_ != nullptr) {
     GpuDeviceScope scope(device_id_);
-    hip_ok(DeviceCache::get().give(device_id_, std::exchange(data_, nullptr), block_), "hipFree");
+    bytes_ = 0;
+    hip_ok(DeviceCache::get().give(device_id_, std::exchange(data_, nullptr),
+                                   std::exchange(block_, 0)),
+           "hipFree");
   }
   bytes_ = 0;
-  block_ = 0;
 }
 
 void GpuDeviceMemory::release_noexcept() noexcept {
@@ -206,11 +224,7 @@ void GpuDeviceMemory::release_noexcept() noexcept {
   int32_t cur = 0;
   const bool switch_dev = gaffa_hip_get_device(&cur) == 0 && cur != device_id_;
   if (switch_dev) (void)gaffa_hip_set_device(device_id_);
-  try {
-    (void)DeviceCache::get().give(device_id_, data_, block_);
-  } catch (...) {  // no memory for the list's node
-    (void)gaffa_hip_free(data_);
-  }
+  (void)DeviceCache::get().give(device_id_, data_, block_);
   if (switch_dev) (void)gaffa_hip_set_device(cur);
   data_ = nullptr;
   bytes_ = 0;
