@@ -22,7 +22,12 @@ except ImportError as exc:  # pragma: no cover - exercised only without a build
         "run `python -m gaffa_amd.build` first"
     ) from exc
 
-from ._core import cuda_device_count, gpu_device_count, gpu_runtime_version  # noqa: E402
+from ._core import (  # noqa: E402
+    cuda_device_count,
+    gpu_device_count,
+    gpu_runtime_version,
+    release_device_cache,
+)
 from . import dedispersion, ffa, io, pipeline, scorer  # noqa: E402
 from .scorer import CandidateScorer  # noqa: E402
 
@@ -38,5 +43,6 @@ __all__ = [
     "gpu_runtime_version",
     "io",
     "pipeline",
+    "release_device_cache",
     "scorer",
 ]

@@ -41,6 +41,9 @@ inline void launch_check(const char* kernel) {
   hip_check(hipGetLastError(), kernel);
 }
 
+// hipMalloc, tried once more where the registered callback makes room.
+void* device_malloc(uint64_t bytes);
+
 template <typename F>
 int guarded(F&& f) {
   try {

@@ -521,8 +521,7 @@ int32_t* error_flag_for_device() {
   hip_check(hipGetDevice(&dev), "hipGetDevice");
   if (dev < 0 || dev >= 64) throw status_error(GAFFA_HIP_RUNTIME, "device ordinal out of range");
   if (flags[dev] == nullptr) {
-    int32_t* p = nullptr;
-    hip_check(hipMalloc(&p, sizeof(int32_t)), "hipMalloc");
+    auto* p = static_cast<int32_t*>(device_malloc(sizeof(int32_t)));
     hip_check(hipMemset(p, 0, sizeof(int32_t)), "hipMemset");
     flags[dev] = p;
   }

@@ -48,8 +48,10 @@ class GpuDeviceScope {
 
 // An owned device allocation.  Released memory is kept for the next allocation
 // of about its size on that device, up to 1/32 of the device's memory (9 GB here);
-// the oldest goes back first, and all of it when an allocation would fail or on
-// release_device_cache().  hipMalloc of memory that was used before costs about
+// the oldest goes back first, and all of it when an allocation of this library
+// (gaffa_hip_malloc and these classes) finds no memory or on
+// release_device_cache(); no other allocator of the process takes it back by
+// itself.  hipMalloc of memory that was used before costs about
 // 24 ms a GB (the driver clears it): a one-shot search of 24 series of 524291
 // samples, 3 GB of workspace, spent 74 of its 85 ms there.  The release waits for
 // the device before a block is kept, as hipFree does, so whatever stream used it

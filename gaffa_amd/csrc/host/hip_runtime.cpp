@@ -19,7 +19,11 @@ class DeviceCache {
  public:
   // Never destroyed: the runtime may be gone before static destructors run.
   static DeviceCache& get() {
-    static DeviceCache* cache = new DeviceCache;
+    static DeviceCache* cache = [] {
+      auto* c = new DeviceCache;
+      (void)gaffa_hip_set_reclaim([](int32_t device) -> int { return get().release(device); });
+      return c;
+    }();
     return *cache;
   }
 
@@ -42,9 +46,7 @@ class DeviceCache {
     }
     void* p = nullptr;
     block = bytes;
-    int status = gaffa_hip_malloc(&p, bytes);
-    if (status != GAFFA_HIP_OK && release(device)) status = gaffa_hip_malloc(&p, bytes);
-    hip_ok(status, "hipMalloc");
+    hip_ok(gaffa_hip_malloc(&p, bytes), "hipMalloc");
     return p;
   }
 

@@ -1,5 +1,6 @@
 // Runtime entry points of the C ABI: device queries, memory, streams,
 // events and graphs.  Thin, checked wrappers over the HIP runtime.
+#include <atomic>
 #include <cstring>
 
 #include "common.hpp"
@@ -7,8 +8,25 @@
 namespace gaffa_hip {
 namespace {
 thread_local std::string g_last_error;
+std::atomic<gaffa_hip_reclaim_fn> g_reclaim{nullptr};
 }
 void set_error(const std::string& message) { g_last_error = message; }
+
+void* device_malloc(uint64_t bytes) {
+  void* p = nullptr;
+  hipError_t err = hipMalloc(&p, bytes);
+  if (err != hipSuccess) {
+    (void)hipGetLastError();  // the next launch check must not see this
+    const gaffa_hip_reclaim_fn reclaim = g_reclaim.load();
+    int dev = 0;
+    if (reclaim != nullptr && hipGetDevice(&dev) == hipSuccess && reclaim(dev) != 0) {
+      err = hipMalloc(&p, bytes);
+      if (err != hipSuccess) (void)hipGetLastError();
+    }
+  }
+  hip_check(err, "hipMalloc");
+  return p;
+}
 }  // namespace gaffa_hip
 
 using namespace gaffa_hip;
@@ -77,11 +95,12 @@ int gaffa_hip_malloc(void** ptr, uint64_t bytes) {
     check(ptr != nullptr, "allocation output must not be null");
     *ptr = nullptr;
     if (bytes == 0) return;
-    const hipError_t err = hipMalloc(ptr, bytes);
-    // a caller may make room and try again: the next launch check must not see this
-    if (err != hipSuccess) (void)hipGetLastError();
-    hip_check(err, "hipMalloc");
+    *ptr = device_malloc(bytes);
   });
+}
+
+int gaffa_hip_set_reclaim(gaffa_hip_reclaim_fn reclaim) {
+  return guarded([&] { g_reclaim.store(reclaim); });
 }
 
 int gaffa_hip_free(void* ptr) {

@@ -65,6 +65,13 @@ int gaffa_hip_set_device(int32_t device);
 int gaffa_hip_get_device(int32_t* device);
 int gaffa_hip_malloc(void** ptr, uint64_t bytes);
 int gaffa_hip_free(void* ptr);
+/* No counterpart in the reference.  `reclaim(device)` is called, with that
+ * device current, when an allocation of this library finds no device memory;
+ * where it returns nonzero (it gave some back) the allocation is tried once
+ * more.  One callback per process (null: none), called by any thread; the host
+ * layer's gives back the memory that it keeps for reuse. */
+typedef int (*gaffa_hip_reclaim_fn)(int32_t device);
+int gaffa_hip_set_reclaim(gaffa_hip_reclaim_fn reclaim);
 /* Copies in any direction (hipMemcpyDefault).  With a NULL stream the copy is
  * synchronous; otherwise it is enqueued on the stream. */
 int gaffa_hip_memcpy(void* dst, const void* src, uint64_t bytes,

@@ -60,8 +60,11 @@ int gaffa_hip_device_info_get(int32_t, gaffa_hip_device_info* out) {
   out->total_memory = kMemory;
   return 0;
 }
+gaffa_hip_reclaim_fn reclaim = nullptr;
+int gaffa_hip_set_reclaim(gaffa_hip_reclaim_fn f) { return reclaim = f, 0; }
 int gaffa_hip_malloc(void** p, uint64_t bytes) {
   *p = nullptr;
+  if (used + bytes > kMemory && reclaim != nullptr) (void)reclaim(current);
   if (used + bytes > kMemory) return GAFFA_HIP_RUNTIME;
   for (auto& l : live)
     if (l.p == nullptr) {
@@ -127,6 +130,11 @@ int main() {
   expect(used <= kMemory / 32 && used > 0, "more kept than the bound, or nothing", 0);
   gaffa::release_device_cache();
   expect(live_count() == 0, "memory lost", 0);
+  // an allocation that needs what is kept gets it
+  current = 31;
+  { gaffa::GpuDeviceMemory kept(kMemory / 40); }
+  { gaffa::GpuDeviceMemory all(kMemory); }
+  expect(used == 0, "more kept than the bound", 0);
   std::printf("%d failures\n", failures);
   return failures < 100 ? failures : 100;
 }

@@ -111,3 +111,32 @@ def test_release_beside_a_capture(gpu):
             lib.gaffa_hip_graph_destroy(graph)
         lib.gaffa_hip_stream_destroy(stream)
         lib.gaffa_hip_free(out)
+
+
+def _free_bytes(lib):
+    import ctypes
+
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_kept_memory_goes_back(gpu):
+    """What is kept is counted as free again after a C-ABI allocation that finds
+    no memory (here more than any device has), and after the public release."""
+    import ctypes
+
+    import gaffa_amd
+
+    lib = ctypes.CDLL(gaffa_amd.HIP_LIBRARY)
+    x = np.random.default_rng(8).integers(1, 99, size=(1, 64 << 20)).astype(np.uint32)  # 256 MB
+    for give_back in ("allocation", "release"):
+        gaffa_amd.release_device_cache()
+        gpu._preprocess_batch_gpu(x, window_samples=None, normalise=False)
+        kept = _free_bytes(lib)
+        if give_back == "allocation":
+            p = ctypes.c_void_p()
+            assert lib.gaffa_hip_malloc(ctypes.byref(p), ctypes.c_uint64(1 << 50)) != 0
+        else:
+            gaffa_amd.release_device_cache()
+        assert _free_bytes(lib) >= kept + x.nbytes, give_back
