@@ -42,7 +42,7 @@ dedisperse_multi_u8_kernel(const uint8_t* __restrict__ x, uint64_t nsamples,
                            uint64_t nchans, uint64_t chan_begin, uint32_t nsel,
                            const int32_t* __restrict__ delays, uint32_t ndm,
                            uint32_t* __restrict__ out, uint64_t out_nsamples,
-                           uint64_t out_stride, uint32_t slab_len,
+                           uint64_t out_stride, uint32_t slab_len, uint32_t slab_rows,
                            int32_t* __restrict__ error_flag) {
   extern __shared__ uint32_t slab32[];
   uint8_t* slab = reinterpret_cast<uint8_t*>(slab32);  // [kBfChans][slab_len]
@@ -81,9 +81,9 @@ dedisperse_multi_u8_kernel(const uint8_t* __restrict__ x, uint64_t nsamples,
     __syncthreads();
     const int32_t dmin = sminmax[0];
     const int32_t spread = sminmax[1] - dmin;
-    // The host sized slab_len from its own table; a mismatch would overrun
+    // The host sized the slab from its own table; a mismatch could overrun
     // LDS, so refuse the block (uniform branch) and report it.
-    if (static_cast<uint32_t>(spread) + kBfTime + 8 > slab_len) {
+    if (static_cast<uint32_t>(spread) + kBfTime + 8 > slab_rows) {
       if (tid == 0) atomicExch(error_flag, 1);
       return;
     }
@@ -590,7 +590,10 @@ int gaffa_hip_dedisperse_multi_u8(const gaffa_hip_dedisperse_multi_args* a,
     check(a->max_block_spread >= 0, "dedispersion requires non-negative delays");
     check(a->ndm <= 0xFFFFFFFFull && a->chan_end - a->chan_begin <= 0xFFFFFFFFull,
           "dedispersion table too large");
-    uint32_t slab_len = static_cast<uint32_t>((kBfTime + a->max_block_spread + 8 + 3) & ~3);
+    // the announced spread's rows, which the kernel holds the delays to
+    const uint32_t slab_rows =
+        static_cast<uint32_t>((kBfTime + a->max_block_spread + 8 + 3) & ~3);
+    uint32_t slab_len = slab_rows;
     // rows 4 bytes past a multiple of 32 keep the staging's writes (8 channels x
     // 8 row groups of a wave) on different banks, where the budget allows it
     const uint32_t padded = slab_len + ((4u - slab_len) & 31u);
@@ -613,7 +616,7 @@ int gaffa_hip_dedisperse_multi_u8(const gaffa_hip_dedisperse_multi_args* a,
                        a->nsamples, a->nchans, a->chan_begin,
                        static_cast<uint32_t>(a->chan_end - a->chan_begin), a->delays,
                        static_cast<uint32_t>(a->ndm), a->out, a->out_nsamples,
-                       a->out_stride, slab_len, error_flag_for_device());
+                       a->out_stride, slab_len, slab_rows, error_flag_for_device());
     launch_check("dedisperse_multi_u8_kernel");
   });
 }

@@ -73,3 +73,38 @@ def test_dedisperse_layouts(gpu, n, nch, begin, end, ndm, spread, offset):
     finally:
         for p in ptrs:
             lib.gaffa_hip_free(p)
+
+
+@pytest.mark.parametrize("announced,spread,ok", [(64, 64, True), (64, 65, False),
+                                                 (64, 92, False), (0, 28, False)])
+def test_understated_spread_is_refused(gpu, announced, spread, ok):
+    """A delay table wider than the announced spread is reported, also where the
+    staging rows' padding (up to 28 samples) would hold it."""
+    import gaffa_amd
+
+    print(f"dedisperse: spread {spread} announced as {announced}", flush=True)
+    lib = ctypes.CDLL(gaffa_amd.HIP_LIBRARY)
+    n, nch = 1024, 32
+    x = np.random.default_rng(spread).integers(0, 256, size=(n, nch), dtype=np.uint8)
+    delays = np.zeros((2, nch), np.int32)
+    delays[1, 3] = spread
+    ptrs = []
+
+    def dev(nbytes):
+        p = ctypes.c_void_p()
+        assert lib.gaffa_hip_malloc(ctypes.byref(p), ctypes.c_uint64(nbytes)) == 0
+        ptrs.append(p)
+        return p
+
+    try:
+        d_x, d_d, d_o = dev(x.nbytes), dev(delays.nbytes), dev(2 * n * 4)
+        for p, host in ((d_x, x), (d_d, delays)):
+            assert lib.gaffa_hip_memcpy(p, host.ctypes.data_as(ctypes.c_void_p),
+                                        ctypes.c_uint64(host.nbytes), None) == 0
+        a = MultiArgs(d_x, n, nch, 0, nch, d_d, 2, d_o, n, n, announced)
+        assert lib.gaffa_hip_dedisperse_multi_u8(ctypes.byref(a), None) == 0
+        assert (lib.gaffa_hip_dedisperse_check(None) == 0) == ok
+        assert lib.gaffa_hip_dedisperse_check(None) == 0  # the report is cleared
+    finally:
+        for p in ptrs:
+            lib.gaffa_hip_free(p)
