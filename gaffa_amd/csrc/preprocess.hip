@@ -292,9 +292,12 @@ detrend_kernel(T* __restrict__ data, uint64_t stride, uint64_t n,
 // every block from their prefix sums, square_map_kernel composes each block's
 // map, and combine_stats_kernel walks the blocks of a series: it applies a map
 // only where S really starts and ends in the map's binade, and else runs the
-// block in finer pieces, down to sample by sample around a binade's end.  Series
-// whose sum can round (or with a sample that is not finite) are left to
-// stats_kernel.
+// block in finer pieces, down to sample by sample around a binade's end.  A batch
+// with a series whose sum can round (or a sample that is not finite) is left to
+// stats_kernel, whose time hardly depends on the number of series:
+// block_exponent_kernel finds it, and neither maps nor walks follow.  Ordinary
+// float series round: 64 of 16384 samples take 211 us in the chain alone, took 291
+// us with the maps and walks before it, and take 219 us without them.
 // The read of the plane bounds square_map_kernel.  Measured, statistics with
 // their part of detrend_kernel: 256 series of 2^20 samples 12.7 -> 0.5 ms, 512
 // of 2^21 25.1 -> 1.2 ms, 128 of 400k 4.8 -> 0.2 ms.
@@ -304,7 +307,8 @@ constexpr uint32_t kMapBlock = kMapThreads * kMapRun;     // smallest block: 409
 constexpr uint32_t kMapMaxShift = 4;                      // blocks of up to 65536 samples
 constexpr int32_t kNoExponent = -1;                       // a block that holds a binade's end
 constexpr int32_t kZeroBlock = -2;                        // a block of zeros
-constexpr int32_t kSerialStats = -1;                      // flags: left to stats_kernel
+constexpr int32_t kSerialStats = INT32_MIN;  // quantum of the batch's first block: left to
+                                             // stats_kernel
 
 // The biased exponent of x >= 0 (zero for a zero).
 __device__ __forceinline__ int32_t exponent_of(double x) {
@@ -337,12 +341,14 @@ __device__ __forceinline__ double read_lane(double x, uint32_t lane) {
   return __builtin_bit_cast(double, lo | (hi << 32));
 }
 
-// sums[b].exponent of every block of a series, a wave per series.
+// sums[b].exponent of every block of a series, and whether its sum can round, a
+// wave per series.
 __global__ void __launch_bounds__(64)
-block_exponent_kernel(BlockSums* __restrict__ sums, uint32_t nblocks) {
+block_exponent_kernel(BlockSums* sums, uint32_t nblocks) {
   BlockSums* const s = sums + static_cast<uint64_t>(blockIdx.x) * nblocks;
   const uint32_t lane = threadIdx.x;
-  double before = 0.0;
+  double before = 0.0, magnitude = 0.0;
+  int32_t quantum = 4096;
   for (uint32_t b0 = 0; b0 < nblocks; b0 += 64) {
     const uint32_t b = b0 + lane;
     const double q = b < nblocks ? static_cast<double>(s[b].squares) : 0.0;
@@ -352,10 +358,23 @@ block_exponent_kernel(BlockSums* __restrict__ sums, uint32_t nblocks) {
       const double x = __shfl_up(upto, off, 64);
       if (lane >= static_cast<uint32_t>(off)) upto += x;
     }
-    if (b < nblocks)
+    if (b < nblocks) {
       s[b].exponent = kept_exponent(before + (upto - q), before + upto, 1e-5);
+      magnitude += static_cast<double>(s[b].magnitude);
+      quantum = min(quantum, s[b].quantum);
+    }
     before += read_lane(upto, 63);
   }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    magnitude += __shfl_xor(magnitude, off, 64);
+    quantum = min(quantum, __shfl_xor(quantum, off, 64));
+  }
+  // multiples of 2^(quantum - 150) that add up to less than 2^53 of them do not
+  // round; a magnitude that is not finite fails.  Where another wave's kSerialStats
+  // is read as the first series' quantum, that series fails too, to the same end.
+  if (lane == 0 && !(magnitude < ldexp(1.0, min(quantum, 400) - 150 + 52)))
+    sums->quantum = kSerialStats;
 }
 
 // maps[series][block]: the block's increments of the sum of squares.
@@ -364,7 +383,7 @@ square_map_kernel(const float* __restrict__ data, uint64_t stride, uint64_t n, u
                   const BlockSums* __restrict__ sums, double2* __restrict__ maps) {
   const uint64_t block = static_cast<uint64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
   const int32_t k = sums[block].exponent;
-  if (k < 0) return;
+  if (k < 0 || sums->quantum == kSerialStats) return;
   const float* x = data + blockIdx.y * stride;
   const uint32_t tid = threadIdx.x;
   const uint64_t i0 = (static_cast<uint64_t>(blockIdx.x) * kMapThreads + tid) * run;
@@ -480,28 +499,14 @@ combine_stats_kernel(const float* __restrict__ data, uint64_t stride, uint64_t n
                      int32_t* __restrict__ status) {
   const uint32_t series = blockIdx.x;
   const uint32_t lane = threadIdx.x;
+  if (sums->quantum == kSerialStats) return;
   const float* x = data + series * stride;
   const BlockSums* const s = sums + static_cast<uint64_t>(series) * nblocks;
   const double2* const f = maps + static_cast<uint64_t>(series) * nblocks;
   SerialSums acc;
-  double magnitude = 0.0;
-  int32_t quantum = 4096;
-  for (uint32_t b = lane; b < nblocks; b += 64) {
-    acc.sum += s[b].sum;
-    magnitude += static_cast<double>(s[b].magnitude);
-    quantum = min(quantum, s[b].quantum);
-  }
+  for (uint32_t b = lane; b < nblocks; b += 64) acc.sum += s[b].sum;
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    acc.sum += __shfl_xor(acc.sum, off, 64);
-    magnitude += __shfl_xor(magnitude, off, 64);
-    quantum = min(quantum, __shfl_xor(quantum, off, 64));
-  }
-  // multiples of 2^(quantum - 150) that add up to less than 2^53 of them
-  if (!(magnitude < ldexp(1.0, min(quantum, 400) - 150 + 52))) {
-    if (lane == 0) flags[series] = kSerialStats;
-    return;
-  }
+  for (int off = 32; off > 0; off >>= 1) acc.sum += __shfl_xor(acc.sum, off, 64);
   constexpr uint32_t kRun = 32;  // samples per lane in a block run in finer pieces
   double S = 0.0;
   for (uint32_t b0 = 0; b0 < nblocks; b0 += 64) {
@@ -563,18 +568,12 @@ combine_stats_kernel(const float* __restrict__ data, uint64_t stride, uint64_t n
   if (lane == 0) finish_stats(acc, n, series, reject_constant, stats, flags, status);
 }
 
-// Whether any of the workgroup's series was left to it (`flagged`: the launch
-// follows combine_stats_kernel; else every series is).
-__device__ __forceinline__ bool any_serial(const int32_t* flags, uint32_t first, uint32_t rows,
-                                           bool flagged) {
-  const uint32_t lane = threadIdx.x & 63u;
-  return !flagged || __ballot(lane < rows && flags[first + lane] == kSerialStats) != 0;
-}
-
 __global__ void __launch_bounds__(kStatsThreads) __attribute__((amdgpu_waves_per_eu(1, 2)))
 stats_kernel(const float* __restrict__ data, uint64_t stride, uint64_t n, uint32_t nseries,
              int32_t reject_constant, double2* __restrict__ stats,
-             int32_t* __restrict__ flags, int32_t* __restrict__ status, bool flagged) {
+             int32_t* __restrict__ flags, int32_t* __restrict__ status,
+             const BlockSums* __restrict__ blocks) {
+  if (blocks != nullptr && blocks->quantum != kSerialStats) return;  // combine_stats_kernel's
   extern __shared__ __align__(16) float stage[];  // [2][kStatsLanes][kStatsPitch]
   __shared__ double squares_of[kStatsLanes];
   const uint32_t tid = threadIdx.x;
@@ -582,7 +581,6 @@ stats_kernel(const float* __restrict__ data, uint64_t stride, uint64_t n, uint32
   const bool squares = tid >= 64u;  // wave-uniform: wave 1 runs the squares
   const uint32_t first = blockIdx.x * kStatsLanes;
   const uint32_t rows = min(static_cast<uint32_t>(kStatsLanes), nseries - first);
-  if (!any_serial(flags, first, rows, flagged)) return;
   const uint64_t nchunks = n / kStatsChunk;
   const float* base = data + static_cast<uint64_t>(first) * stride;
   // load k of a chunk: element e = k * 128 + tid is row e / kStatsVecs,
@@ -674,11 +672,10 @@ stats_kernel(const float* __restrict__ data, uint64_t stride, uint64_t n, uint32
 __global__ void __launch_bounds__(kStatsLanes)
 stats_rowwise_kernel(const float* __restrict__ data, uint64_t stride, uint64_t n,
                      uint32_t nseries, int32_t reject_constant, double2* __restrict__ stats,
-                     int32_t* __restrict__ flags, int32_t* __restrict__ status, bool flagged) {
-  const uint32_t first = blockIdx.x * kStatsLanes;
-  const uint32_t series = first + threadIdx.x;
-  if (!any_serial(flags, first, min(static_cast<uint32_t>(kStatsLanes), nseries - first), flagged))
-    return;
+                     int32_t* __restrict__ flags, int32_t* __restrict__ status,
+                     const BlockSums* __restrict__ blocks) {
+  if (blocks != nullptr && blocks->quantum != kSerialStats) return;  // combine_stats_kernel's
+  const uint32_t series = blockIdx.x * kStatsLanes + threadIdx.x;
   if (series >= nseries) return;
   const float* x = data + static_cast<uint64_t>(series) * stride;
   SerialSums acc;
@@ -856,12 +853,12 @@ void run(const gaffa_hip_preprocess_args* a, void* workspace, hipStream_t st) {
                 "hipFuncSetAttribute");
       hipLaunchKernelGGL(stats_kernel, sg, dim3(kStatsThreads), kStatsLdsBytes, st, fdata,
                          a->stride, a->nsamples, static_cast<uint32_t>(a->nseries),
-                         a->reject_constant, stats, flags, a->status, sb.on);
+                         a->reject_constant, stats, flags, a->status, sb.sums);
       launch_check("stats_kernel");
     } else {
       hipLaunchKernelGGL(stats_rowwise_kernel, sg, dim3(kStatsLanes), 0, st, fdata, a->stride,
                          a->nsamples, static_cast<uint32_t>(a->nseries), a->reject_constant,
-                         stats, flags, a->status, sb.on);
+                         stats, flags, a->status, sb.sums);
       launch_check("stats_rowwise_kernel");
     }
     hipLaunchKernelGGL(normalise_kernel, g, dim3(kThreads), 0, st,

@@ -94,3 +94,48 @@ def test_statistics_equal_sums_in_sample_order(gpu, kind):
         var = np.cumsum(d * d, axis=1)[:, -1] / n - mean * mean
         np.testing.assert_array_equal(got[:, 0], mean)
         np.testing.assert_array_equal(got[:, 1], 1.0 / np.sqrt(var))
+
+
+def _normalise(x, sentinel):
+    """Normalises x in place on the device with a workspace of `sentinel` bytes;
+    the workspace afterwards."""
+    import gaffa_amd
+
+    lib = ctypes.CDLL(gaffa_amd.HIP_LIBRARY)
+    f = lib.gaffa_hip_preprocess_workspace_bytes
+    f.restype, f.argtypes = ctypes.c_uint64, [ctypes.c_uint64] * 3
+    ns, n = x.shape
+    work = np.full(f(ns, n, 1), sentinel, np.uint8)
+    status = np.zeros(ns, np.int32)
+    ptrs = []
+    try:
+        for host in (x, work, status):
+            p = ctypes.c_void_p()
+            assert lib.gaffa_hip_malloc(ctypes.byref(p), ctypes.c_uint64(host.nbytes)) == 0
+            ptrs.append(p)
+            assert lib.gaffa_hip_memcpy(p, host.ctypes.data_as(ctypes.c_void_p),
+                                        ctypes.c_uint64(host.nbytes), None) == 0
+        a = PreprocessArgs(ptrs[0], ns, n, n, 0, 0, 1, 1, 1, 1, ptrs[1], work.nbytes, ptrs[2])
+        assert lib.gaffa_hip_detrend_normalise_batch(ctypes.byref(a), None) == 0
+        assert lib.gaffa_hip_memcpy(work.ctypes.data_as(ctypes.c_void_p), ptrs[1],
+                                    ctypes.c_uint64(work.nbytes), None) == 0
+        return work
+    finally:
+        for p in ptrs:
+            lib.gaffa_hip_free(p)
+
+
+def test_no_maps_where_the_serial_chain_runs(gpu):
+    """One series whose plain sum rounds sends its batch to the serial chain, and no
+    maps are built for it (the workspace behind the block sums stays as it was)."""
+    rng = np.random.default_rng(3)
+    ns, n, blocks = 66, 3 * 4096 + 5, 4
+    x = np.stack([_series("integers", n, rng) for _ in range(ns)]).astype(np.float32)
+    at = (ns * blocks * 24 + 15) // 16 * 16
+    for rounds in (None, 0, 65):
+        y = x.copy()
+        if rounds is not None:
+            y[rounds, 7] = 2.0 ** -60
+        print(f"maps: series that rounds {rounds}", flush=True)
+        maps = _normalise(y, 0xCD)[at:at + 16 * ns * blocks]
+        assert (maps == 0xCD).all() == (rounds is not None)
