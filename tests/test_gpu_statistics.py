@@ -139,3 +139,38 @@ def test_no_maps_where_the_serial_chain_runs(gpu):
         print(f"maps: series that rounds {rounds}", flush=True)
         maps = _normalise(y, 0xCD)[at:at + 16 * ns * blocks]
         assert (maps == 0xCD).all() == (rounds is not None)
+
+
+def _block_shift(ns, n, factor):
+    """Blocks of 4096 << shift samples: the first whose sums (24 bytes a block) and
+    maps (16) fit the low-resolution series and the medians that they replace; None
+    where none does and every series runs in the serial chain."""
+    low = 4 * ns * (n // factor)
+    for shift in range(5):
+        blocks = ns * -(-n // (4096 << shift))
+        if 24 * blocks <= low and (low + 15) // 16 * 16 + 16 * blocks <= 2 * low:
+            return shift
+    return None
+
+
+def test_statistics_in_every_block_size(gpu, port):
+    """Detrended and normalised series equal the oracle's bit for bit on both sides of
+    each scrunch factor at which the blocks of the statistics double (whose sums then
+    fill the scratch to the last byte), and past the last one; a last block that is
+    nearly full, and one that is not; whole numbers, and floats whose sum rounds."""
+    rng = np.random.default_rng(11)
+    seen = set()
+    for n in (96 * 4096 - 5, 300001):
+        for factor in (2, 682, 683, 1365, 1366, 2730, 2731, 5461, 5462, 10922, 10923):
+            whole = n != 300001 or factor % 2 == 0
+            x = rng.integers(0, 4000, size=(3, n)) if whole else rng.normal(size=(3, n))
+            x = x.astype(np.uint32 if whole else np.float32)
+            seen.add(_block_shift(3, n, factor))
+            print(f"statistics: factor {factor}, {n} samples, block shift "
+                  f"{_block_shift(3, n, factor)}", flush=True)
+            window = (5 * factor) | 1
+            got = gpu._preprocess_batch_gpu(x, window_samples=window, min_points=5)
+            for i in range(3):
+                want = port.normalise(port.detrend(x[i].astype(np.float32), window, 5))
+                np.testing.assert_array_equal(got[i], want)
+    assert seen == {0, 1, 2, 3, 4, None}
