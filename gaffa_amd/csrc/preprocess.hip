@@ -747,7 +747,8 @@ Layout layout(uint64_t nseries, uint64_t n, uint64_t factor) {
 // free once its medians are taken, and the medians once they are subtracted, so
 // blocks of kMapBlock << shift samples live there and need no room of their own.
 // Off where they do not fit (scrunch factors past 10^4, an exact running median,
-// which leaves no low-resolution series): stats_kernel then runs every series.
+// which leaves no low-resolution series) and for short series: stats_kernel then
+// runs every series.
 struct StatsBlocks {
   bool on = false;
   uint32_t shift = 0;
@@ -759,6 +760,12 @@ struct StatsBlocks {
 StatsBlocks stats_blocks(const gaffa_hip_preprocess_args* a, const Layout& l, void* workspace) {
   StatsBlocks s;
   if (!a->normalise || (a->detrend && a->scrunch_factor == 1)) return s;
+  // Three launches more than the chain, which takes 12 ns a sample: chain -> blocks,
+  // us, of whole numbers 1 x 1024 samples 21 -> 30, 1024 x 1024 26 -> 35, 1 x 2048
+  // 35 -> 32, 1024 x 2048 42 -> 41.  Floats, whose batch may end in the chain: 1024 x
+  // 2048 42 -> 55 (there), 1 x 2048 35 -> 35, 1 x 4096 59 -> 44, 1024 x 4096 73 -> 85
+  // (there).
+  if (a->nsamples < (a->input_is_u32 ? 2048u : 4096u)) return s;
   auto align = [](uint64_t v) { return (v + 15) / 16 * 16; };
   const uint64_t end = (l.low_floats + l.med_floats) * 4;
   for (uint32_t shift = 0; shift <= kMapMaxShift; ++shift) {

@@ -115,7 +115,8 @@ def _normalise(x, sentinel):
             ptrs.append(p)
             assert lib.gaffa_hip_memcpy(p, host.ctypes.data_as(ctypes.c_void_p),
                                         ctypes.c_uint64(host.nbytes), None) == 0
-        a = PreprocessArgs(ptrs[0], ns, n, n, 0, 0, 1, 1, 1, 1, ptrs[1], work.nbytes, ptrs[2])
+        a = PreprocessArgs(ptrs[0], ns, n, n, int(x.dtype == np.uint32), 0, 1, 1, 1, 1, ptrs[1],
+                           work.nbytes, ptrs[2])
         assert lib.gaffa_hip_detrend_normalise_batch(ctypes.byref(a), None) == 0
         assert lib.gaffa_hip_memcpy(work.ctypes.data_as(ctypes.c_void_p), ptrs[1],
                                     ctypes.c_uint64(work.nbytes), None) == 0
@@ -174,3 +175,14 @@ def test_statistics_in_every_block_size(gpu, port):
                 want = port.normalise(port.detrend(x[i].astype(np.float32), window, 5))
                 np.testing.assert_array_equal(got[i], want)
     assert seen == {0, 1, 2, 3, 4, None}
+
+
+@pytest.mark.parametrize("dtype,least", [(np.uint32, 2048), (np.float32, 4096)])
+def test_short_series_run_the_serial_chain(gpu, dtype, least):
+    """Series below the length at which blocks pay run in the serial chain alone: the
+    workspace in front of the statistics stays as it was."""
+    rng = np.random.default_rng(4)
+    for ns, n in ((1, least - 1), (65, least - 1), (1, least)):
+        x = rng.integers(1, 4000, size=(ns, n)).astype(dtype)
+        print(f"short series: {ns} x {n} {np.dtype(dtype)}", flush=True)
+        assert (_normalise(x, 0xCD)[:4 * ns * n] == 0xCD).all() == (n < least)
