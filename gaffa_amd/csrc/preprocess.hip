@@ -60,8 +60,18 @@ scrunch_kernel(const T* __restrict__ data, uint64_t stride, uint64_t factor,
 // loads into LDS, and `lanes` (a power of two) neighbouring lanes sum one
 // output.  The read of the plane bounds it: a wave per output left lanes idle
 // at f = 38 and had one load in flight each.  128 series x 400k samples, f = 38
-// (205 MB): 226 us before, 57 us now, 3.6 TB/s.
+// (205 MB): 226 us before, 57 us now, 3.6 TB/s.  Fewer outputs a workgroup where
+// kScrunchGroups of them would not be reached: detrending one series of 16384
+// samples at f = 2 takes 39 us so, 44 us with 4 full workgroups.
 constexpr uint32_t kScrunchSpan = 4096;
+constexpr uint32_t kScrunchGroups = 1024;
+// Past this factor a wave per output keeps all lanes busy and is the faster one
+// where its waves fill the chip.  Detrending, wave per output against spans, us: 16
+// series of 2^20 samples at f = 104 108, 97; 256 92, 89; 309 91, 94; 700 86, 92; one
+// series at f = 309 (3393 outputs) 43, 44; at 1000 (1048 outputs) 42, 41; at 3000
+// (349) 55, 47.
+constexpr uint32_t kScrunchWave = 256;
+constexpr uint32_t kScrunchWaveOutputs = 2048;
 
 __global__ void __launch_bounds__(kThreads)
 scrunch_u32_kernel(const uint32_t* __restrict__ data, uint64_t stride, uint32_t factor,
@@ -91,7 +101,7 @@ scrunch_u32_kernel(const uint32_t* __restrict__ data, uint64_t stride, uint32_t 
   }
 }
 
-// The same for factors past kScrunchSpan: one wave per output, shuffle reduction.
+// The same with one wave per output and a shuffle reduction.
 __global__ void __launch_bounds__(kThreads)
 scrunch_u32_wide_kernel(const uint32_t* __restrict__ data, uint64_t stride, uint64_t factor,
                         uint64_t m, float* __restrict__ low) {
@@ -805,8 +815,10 @@ void run(const gaffa_hip_preprocess_args* a, void* workspace, hipStream_t st) {
   if (a->detrend) {
     if (f > 1) {
       if constexpr (std::is_same_v<T, uint32_t>) {
-        if (f <= kScrunchSpan) {
-          const uint32_t outputs = kScrunchSpan / static_cast<uint32_t>(f);
+        const uint64_t all = a->nseries * l.m;
+        if (f <= kScrunchSpan && (f <= kScrunchWave || all < kScrunchWaveOutputs)) {
+          const uint32_t outputs = static_cast<uint32_t>(std::min<uint64_t>(
+              kScrunchSpan / f, std::max<uint64_t>(1, all / kScrunchGroups)));
           uint32_t lanes = 1;  // about one output per group of lanes
           while (lanes < 64 && 2 * lanes * outputs <= kThreads) lanes *= 2;
           const dim3 g(static_cast<uint32_t>(ceil_div(l.m, outputs)),

@@ -21,3 +21,25 @@ def test_scrunch_factors(gpu, port, factor):
     for i in range(3):
         want = port.detrend(x[i].astype(np.float32), window, 5)
         np.testing.assert_array_equal(got[i], want)
+
+
+@pytest.mark.parametrize("factor,ns,outputs", [
+    (2, 5, 430001),     # as many outputs a workgroup as LDS holds, the last one partly full
+    (38, 9, 14001),     # the same
+    (256, 7, 300),      # 2 of 16
+    (256, 3, 6001),     # 16
+    (257, 7, 292),      # spans (2044 outputs) ...
+    (257, 7, 293),      # ... and a wave per output (2051)
+    (1000, 23, 101),
+])
+def test_scrunch_outputs(gpu, port, factor, ns, outputs):
+    """Both sides of the lines between fewer and more outputs a workgroup and between
+    spans and a wave per output."""
+    rng = np.random.default_rng(factor + outputs)
+    n = factor * outputs + factor // 3
+    print(f"scrunch: factor {factor}, {ns} series x {n}", flush=True)
+    x = rng.integers(0, 60000, size=(ns, n)).astype(np.uint32)
+    window = (5 * factor) | 1
+    got = gpu._preprocess_batch_gpu(x, window_samples=window, min_points=5, normalise=False)
+    for i in range(ns):
+        np.testing.assert_array_equal(got[i], port.detrend(x[i].astype(np.float32), window, 5))
