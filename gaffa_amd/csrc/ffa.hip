@@ -13,11 +13,13 @@
 //             loads, then each output is summed serially in the CPU's FP32
 //             order
 //   subtree   persistent workgroups walking (node at the task's LDS depth D,
-//             series) units.  Plans of up to 304 bins: two workgroups per CU,
-//             each wave runs one of the node's eight sub-nodes in registers
-//             and the top three levels merge from LDS.  Other plans: one
-//             workgroup per CU, every level in LDS between two buffers, with
-//             merges from host-built tables
+//             series) units.  Plans of up to 304 bins and 160 rows a node:
+//             two workgroups per CU, each wave runs one of the node's eight
+//             sub-nodes in registers and the top three levels merge from
+//             LDS.  Other plans, as a whole (one larger node is enough), and
+//             those mostly of nodes below 64 bins: one workgroup per CU, every
+//             level in LDS between two buffers, with merges from host-built
+//             tables
 //   level     one launch per output depth: one to three levels per pass,
 //             each item (32 rows of one node) copying its leaf rows' runs
 //             from HBM into LDS and merging there
@@ -647,8 +649,9 @@ ffa_subtree_kernel(KArgs a, uint32_t nunits) {
 // -------------------------------------------------- subtree, registers ----
 // The subtree kernel of plans whose nodes all hold at most kNodeMaxRows rows of
 // at most kNodeMaxBins bins: beyond them a sub-node no longer fits 64 registers
-// per lane (rows x C), and ffa_subtree_kernel runs the plan.  A 512-thread workgroup runs one (node, series) unit
-// at a time, two workgroups per CU:
+// per lane (rows x C), and ffa_subtree_kernel runs the plan, as it does where most
+// nodes are too small for registers (subtree_gain).  A 512-thread workgroup runs
+// one (node, series) unit at a time, two workgroups per CU:
 //   1. wave w owns the node's depth-3 sub-node w (ceil(rows / 8) rows at most)
 //      and runs all of its levels in registers.  Lane l holds phases l C ..
 //      l C + C - 1 of every row (the phases past the row's end being its
@@ -1554,6 +1557,26 @@ bool nodes_in_registers(const gaffa_hip_ffa_plan_desc& p) {
   return p.max_bins <= kNodeMaxBins && p.max_subtree_desc <= subtree_entries(kNodeMaxRows);
 }
 
+// Whether ffa_node_kernel runs the plan: where it can, and the builder did not find
+// the tables' kernel faster.
+bool uses_node_kernel(const gaffa_hip_ffa_plan_desc& p) {
+  return nodes_in_registers(p) && (p.subtree_from_tables == 0 || p.subtree_merges == nullptr);
+}
+
+// Nodes without registers (few bins or rows, node_regs_per_row) run level by level
+// in ffa_node_kernel, and their time grows with floats x levels; with tables it
+// hardly grows with the bins.  Measured, 1024 nodes a launch, tables -> registers or
+// levels: 63 bins x 12 rows 19 -> 16 us, x 24 24 -> 31, x 160 68 -> 265; 24 bins x 48
+// 30 -> 30, x 160 65 -> 105; 300 bins x 4 rows 16 -> 14, x 7 21 -> 26; in registers 64
+// bins x 8 16 -> 9, x 160 68 -> 32, 256 bins x 64 49 -> 31.  The lines through those,
+// in 1/300 us: levels 1800 + floats levels, tables 4200 + 100 rows, and what
+// registers save 2100 + 45 rows.
+int64_t subtree_gain(uint32_t rows, uint32_t bins) {
+  const int64_t r = rows;
+  if (node_regs_per_row(rows, bins) != 0) return 2100 + 45 * r;
+  return 2400 + 100 * r - r * bins * tree_levels(rows);
+}
+
 // Leaf rows of 8 level items a workgroup, a thread per row: stores bound it (36 MB
 // at 2^22 samples).  On the host, with the merge tables that plans in registers
 // never read, they were most of a one-shot search of one such series: 23 ms of
@@ -1598,7 +1621,7 @@ void validate(const gaffa_hip_ffa_search_args* a) {
   check(p.nsubtree_items == 0 ||
             (p.subtree_half_floats > 0 &&
              p.subtree_half_floats <= kSubtreePrefetch * kSubtreeThreads &&
-             (p.subtree_merges != nullptr || p.max_subtree_desc == 0 || nodes_in_registers(p)) &&
+             (p.subtree_merges != nullptr || p.max_subtree_desc == 0 || uses_node_kernel(p)) &&
              8ull * p.subtree_half_floats + 4ull * kSubtreeGuard +
                      4ull * subtree_zero_floats(p.max_bins) <= p.subtree_lds_bytes),
         "FFA subtree geometry inconsistent");
@@ -1673,7 +1696,7 @@ void launch_subtrees(const gaffa_hip_ffa_search_args* a, hipStream_t st) {
   if (p.nsubtree_items > 0) {
     const uint64_t nunits = static_cast<uint64_t>(p.nsubtree_items) * ns;
     check_overflow(nunits < (1ull << 32), "FFA subtree work too large");
-    if (nodes_in_registers(p)) {
+    if (uses_node_kernel(p)) {
       const uint32_t bytes = node_lds_bytes(p.subtree_half_floats);
       ensure_dynamic_lds(reinterpret_cast<const void*>(ffa_node_kernel), 4, bytes);
       const uint32_t grid = static_cast<uint32_t>(
@@ -1791,7 +1814,7 @@ int gaffa_hip_ffa_reserve_launch(const gaffa_hip_ffa_plan_desc* p) {
     check(p->subtree_lds_bytes <= kMaxLdsBytes && p->terminal_lds_bytes <= kMaxLdsBytes &&
               p->level_lds_bytes <= kMaxLevelLdsBytes,
           "FFA plan exceeds LDS");
-    if (p->nsubtree_items > 0 && nodes_in_registers(*p))
+    if (p->nsubtree_items > 0 && uses_node_kernel(*p))
       ensure_dynamic_lds(reinterpret_cast<const void*>(ffa_node_kernel), 4,
                          node_lds_bytes(p->subtree_half_floats));
     else if (p->nsubtree_items > 0)
@@ -1823,6 +1846,10 @@ int gaffa_hip_ffa_build_level_rows(const gaffa_hip_ffa_task* tasks,
 
 uint32_t gaffa_hip_ffa_subtree_reads_merges(uint32_t max_rows, uint32_t max_bins) {
   return max_rows > kNodeMaxRows || max_bins > kNodeMaxBins ? 1u : 0u;
+}
+
+int64_t gaffa_hip_ffa_subtree_gain(uint32_t rows, uint32_t bins) {
+  return subtree_gain(rows, bins);
 }
 
 uint32_t gaffa_hip_ffa_prepare_outputs_per_block(double factor) {

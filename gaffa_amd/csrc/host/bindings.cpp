@@ -735,6 +735,8 @@ PYBIND11_MODULE(_core, m) {
         d["spans"] = words(e.level_spans(), 20);
         d["leaf_rows"] = words(e.level_leaf_rows(), 16);
         d["level_lds_bytes"] = e.level_lds_bytes();
+        d["subtree_merges"] = e.subtree_merges().size();
+        d["subtree_from_tables"] = e.subtree_from_tables();
         return d;
       },
       py::arg("plan"), py::arg("level_rows") = 0,

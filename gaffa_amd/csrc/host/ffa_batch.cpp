@@ -136,6 +136,7 @@ void GpuFfaBatchedSearch::build_tiles() {
     d.ntasks = static_cast<std::uint32_t>(e.tasks().size());
     d.subtree_items = t->subtree.data();
     d.nsubtree_items = static_cast<std::uint32_t>(e.subtree_items().size());
+    d.subtree_from_tables = e.subtree_from_tables() ? 1 : 0;
     d.subtree_merges = t->merges.data();
     d.level_items = t->level.data();
     d.level_spans = t->level_spans.data();

@@ -134,21 +134,28 @@ std::uint32_t GpuFfaExecutionPlan::lds_depth(std::size_t rows, std::size_t bins)
   return depth;
 }
 
-// Whether some node is beyond the kernel that reads no merge tables; tasks that
-// append() refuses do not matter here.
+// Whether some node is beyond the kernel that reads no merge tables, or the nodes
+// together lose in it; tasks that append() refuses do not matter here.
 void GpuFfaExecutionPlan::find_needs_merges(std::span<const FfaSearchPlan* const> plans) {
   if (subtree_fixed_lds(lds_max_bins_) >= kSubtreeLdsBytes) return;
   const std::size_t node_floats = (kSubtreeLdsBytes - subtree_fixed_lds(lds_max_bins_)) / 8;
   std::size_t most = 0;
+  std::int64_t gain = 0;
   for (const FfaSearchPlan* plan : plans)
     for (const FfaSearchTask& t : plan->tasks) {
       if (t.rows < 2 || t.bins < 2 || t.rows >= (std::size_t{1} << 31) || node_floats / t.bins < 2)
         continue;
       const std::uint32_t depth = lds_depth(t.rows, t.bins);
-      most = std::max(most, (t.rows + (std::size_t{1} << depth) - 1) >> depth);
+      const std::size_t rows = (t.rows + (std::size_t{1} << depth) - 1) >> depth;
+      most = std::max(most, rows);
+      gain += (std::int64_t{1} << depth) *
+              gaffa_hip_ffa_subtree_gain(static_cast<std::uint32_t>(rows),
+                                         static_cast<std::uint32_t>(t.bins));
     }
   needs_merges_ = gaffa_hip_ffa_subtree_reads_merges(static_cast<std::uint32_t>(most),
                                                      static_cast<std::uint32_t>(lds_max_bins_)) != 0;
+  from_tables_ = !needs_merges_ && gain < 0;
+  needs_merges_ = needs_merges_ || from_tables_;
 }
 
 GpuDeviceBuffer<gaffa_hip_ffa_level_row> GpuFfaExecutionPlan::build_level_leaf_rows(
@@ -433,6 +440,7 @@ GpuFfaProgram::GpuFfaProgram(const FfaSearchPlan& plan, const GpuFfaProgramOptio
   desc_.ntasks = static_cast<std::uint32_t>(t.size());
   desc_.subtree_items = d_subtree_.data();
   desc_.nsubtree_items = static_cast<std::uint32_t>(exec_plan_.subtree_items().size());
+  desc_.subtree_from_tables = exec_plan_.subtree_from_tables() ? 1 : 0;
   desc_.subtree_merges = d_merges_.data();
   desc_.level_items = d_level_.data();
   desc_.level_spans = d_level_spans_.data();

@@ -102,6 +102,8 @@ class GpuFfaExecutionPlan {
   std::uint32_t subtree_lds_bytes() const noexcept { return subtree_lds_bytes_; }
   std::uint32_t subtree_half_floats() const noexcept { return subtree_half_; }
   std::uint32_t max_subtree_desc() const noexcept { return subtree_desc_; }
+  // the kernel that reads the merge tables is the faster of two that can run this
+  bool subtree_from_tables() const noexcept { return from_tables_; }
   std::uint32_t terminal_lds_bytes() const noexcept { return terminal_lds_bytes_; }
   std::uint32_t level_lds_bytes() const noexcept { return level_lds_bytes_; }
   std::uint32_t prep_blocks() const noexcept { return prep_blocks_; }
@@ -128,6 +130,7 @@ class GpuFfaExecutionPlan {
   std::size_t max_prepared_ = 0;
   std::size_t lds_max_bins_ = 0;  // bins of the widest task of every plan appended
   bool needs_merges_ = true;      // the subtree kernel reads the merge tables
+  bool from_tables_ = false;      // ... by choice
   // rows of a subtree node in LDS, and the depth of the first nodes that fit
   std::size_t lds_rows(std::size_t bins) const;
   std::uint32_t lds_depth(std::size_t rows, std::size_t bins) const;

@@ -427,6 +427,9 @@ typedef struct gaffa_hip_ffa_plan_desc {
   uint32_t ntasks;
   const gaffa_hip_ffa_item* subtree_items; /* device; c = first merge */
   uint32_t nsubtree_items;
+  uint32_t subtree_from_tables; /* nonzero: with the kernel that reads the merge
+                                  tables, also where ..._subtree_reads_merges()
+                                  says 0 (..._subtree_gain() below 0) */
   const gaffa_hip_ffa_merge* subtree_merges; /* device; may be null where
                                   ..._subtree_reads_merges() says 0 */
   const gaffa_hip_ffa_item* level_items;   /* device, sorted by depth desc */
@@ -506,6 +509,10 @@ uint32_t gaffa_hip_ffa_subtree_lds_bytes(uint32_t rows, uint32_t bins);
  * at most `max_bins` bins reads the merge tables; else subtree_merges may be null
  * (max_subtree_desc is the tables' size all the same). */
 uint32_t gaffa_hip_ffa_subtree_reads_merges(uint32_t max_rows, uint32_t max_bins);
+/* What one node of `rows` rows of `bins` bins gains in the kernel that reads no
+ * merge tables over the one that does, in units of its own (negative: it loses);
+ * for the choice of a plan that either can run, over the sum of its nodes. */
+int64_t gaffa_hip_ffa_subtree_gain(uint32_t rows, uint32_t bins);
 /* Fills the merge table of a subtree node of `rows` rows (host memory; a
  * null `out` only counts) with the kernels' own row-selection arithmetic
  * (gaffa's ffa.cpp:133-143 in FP32).  Returns the entry count, 0 for rows

@@ -583,3 +583,45 @@ def test_bench_refuses_more_than_one_gpu():
                        capture_output=True, text=True, timeout=120)
     assert r.returncode == 2
     assert "measures one GPU" in r.stderr and r.stdout == ""
+
+
+@pytest.mark.parametrize("nsamples,bins_min,bins_max,periods,tables", [
+    (18000, 60, 63, (0.0601, 2.0), True),    # nodes of up to 150 rows of fewer than 64 bins
+    (9000, 32, 46, (0.033, 0.4), True),
+    (600, 8, 12, (0.01, 0.1), False),        # so small that tables do not pay
+    (4000, 32, 46, (0.033, 0.4), False),
+    (20000, 64, 80, (0.0641, 1.0), False),   # in registers
+    (30000, 180, 256, (0.2, 2.0), False),
+    (2900, 180, 256, (0.2, 0.7), False),     # rows too few for registers
+])
+def test_small_nodes_choose_their_subtree_kernel(nsamples, bins_min, bins_max, periods, tables):
+    """Plans that either subtree kernel can run take the one that reads merge tables
+    where their nodes together are faster with it: many rows of fewer than 64 bins."""
+    from gaffa_amd import _core as core
+    from gaffa_amd.ffa import make_riptide_plan
+
+    plan = make_riptide_plan(nsamples=nsamples, tsamp=1e-3, period_min=periods[0],
+                             period_max=periods[1], bins_min=bins_min, bins_max=bins_max)
+    d = core._ffa_level_layout(plan)
+    assert d["subtree_from_tables"] == tables
+    assert (d["subtree_merges"] > 0) == tables
+
+
+def test_subtree_gain_follows_the_measured_nodes():
+    """The rule's sign against node times measured with 1024 nodes a launch (tables,
+    the other kernel; us), where the two differ by 10 % or more."""
+    import ctypes
+
+    import gaffa_amd
+
+    gain = ctypes.CDLL(gaffa_amd.HIP_LIBRARY).gaffa_hip_ffa_subtree_gain
+    gain.restype, gain.argtypes = ctypes.c_int64, [ctypes.c_uint32, ctypes.c_uint32]
+    for bins, rows, tables, other in (
+            (8, 160, 64.3, 41.8), (16, 80, 42.2, 35.9), (16, 160, 64.6, 74.9), (24, 24, 23.5, 17.6),
+            (24, 80, 42.5, 53.1), (32, 24, 23.1, 19.2), (32, 48, 30.4, 36.4), (32, 160, 65.3, 137.4),
+            (40, 12, 17.9, 12.6), (40, 48, 30.6, 45.5), (48, 12, 18.0, 15.1), (48, 48, 30.6, 49.0),
+            (56, 12, 18.2, 16.3), (56, 24, 23.6, 29.2), (63, 12, 18.6, 16.0), (63, 24, 24.2, 30.9),
+            (63, 160, 68.0, 265.2), (100, 7, 16.9, 13.3), (200, 4, 14.1, 11.5), (300, 4, 16.0, 13.6),
+            (300, 7, 20.9, 26.0), (64, 8, 16.4, 9.0), (64, 160, 68.4, 32.0), (126, 160, 83.7, 44.6),
+            (193, 104, 74.0, 48.0), (256, 78, 63.6, 37.8), (304, 66, 77.4, 37.6)):
+        assert (gain(rows, bins) > 0) == (other < tables), (bins, rows)
