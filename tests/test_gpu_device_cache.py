@@ -1,6 +1,7 @@
 """GPU: device memory kept between calls never carries one call into another."""
 
 import threading
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -27,29 +28,24 @@ def test_reused_device_memory_keeps_results(gpu):
         gpu.release_device_cache()
         jobs.append((x, plan, _peaks(ffa_search_batch(x, plan))))
         assert jobs[-1][2]
-    bad = []
 
     def work(order):
-        for k in order:
-            x, plan, want = jobs[k]
-            if _peaks(ffa_search_batch(x, plan)) != want:
-                bad.append(k)
+        """The jobs that gave something else; a call that fails raises in result()."""
+        return [k for k in order if _peaks(ffa_search_batch(*jobs[k][:2])) != jobs[k][2]]
 
-    work([0, 1, 2, 1, 0])
-    threads = [threading.Thread(target=work, args=(o,)) for o in ([0, 1, 2] * 4, [2, 0, 1] * 4)]
-    for t in threads:
-        t.start()
-    for t in threads:
-        t.join()
+    assert work([0, 1, 2, 1, 0]) == []
+    with ThreadPoolExecutor(2) as pool:
+        both = [pool.submit(work, o) for o in ([0, 1, 2] * 4, [2, 0, 1] * 4)]
+        assert [f.result() for f in both] == [[], []]
     gpu.release_device_cache()
-    work([2, 1, 0])
-    assert bad == []
+    assert work([2, 1, 0]) == []
 
 
 def test_gradient_padding_is_zero_in_used_memory(gpu):
     """The parameter vector is padded to a multiple of 8; its gradient there is
     zero, also where the scorer's buffers held another call's data before."""
     import gaffa_amd
+    from gaffa_amd.ffa import FfaBatchedSearch, make_riptide_plan
     from oracle import scorer_oracle as so
 
     gpu.release_device_cache()
@@ -60,13 +56,15 @@ def test_gradient_padding_is_zero_in_used_memory(gpu):
     def leave():
         for _ in range(4):
             gpu._preprocess_batch_gpu(x, window_samples=None, normalise=True)
+        return True
 
-    threads = [threading.Thread(target=leave) for _ in range(6)]
     gpu.release_device_cache()
-    for t in threads:
-        t.start()
-    for t in threads:
-        t.join()
+    with ThreadPoolExecutor(6) as pool:
+        assert all(f.result() for f in [pool.submit(leave) for _ in range(6)])
+    # an allocation of the parameters' size gets one of the blocks, as it was left
+    plan = make_riptide_plan(nsamples=size, tsamp=1e-3, period_min=1.0, period_max=1.1)
+    row = FfaBatchedSearch([plan]).download_row()
+    assert size <= row.size <= x.size and (row[:size] != 0).all()
     s = gaffa_amd.CandidateScorer(capacity=8)
     _, g = s.gradients(rng.normal(size=(8, so.SUBINTS, so.PHASE)).astype(np.float32),
                        rng.normal(size=(8, so.PATCH)).astype(np.float32),
