@@ -1,14 +1,11 @@
-"""Level passes whose items exceed the launch's LDS: not yet run on a GPU, so
-kept under a name pytest does not collect.  Run it by naming the file:
-
-    python -u -m pytest tests/wip_level_fallback.py -m gpu -x -v --timeout 120 \
-        --timeout-method thread
+"""GPU: level passes whose items exceed the launch's LDS.
 
 At 800 bins every 32-row item of a three- or two-level pass stages more
 than 64 KB of leaf rows, so the plan gives the level launch no LDS and every
 item merges from global memory (clamped phases, the same FP32 sum tree); at
-400 bins some items fit and some do not, so one launch takes both paths.
-The detection tiles still fit.  The transform rows must equal the oracle's
+1500 rows of 440 bins half of the three-level pass's items need up to 71 424
+bytes and half fit (at 400 bins all would: 65 024 at most), so one launch takes
+both paths.  The detection tiles still fit.  The transform rows must equal the oracle's
 bit for bit.
 """
 
@@ -21,7 +18,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("rows_bins", [(600, 800), (1500, 400)])
+@pytest.mark.parametrize("rows_bins", [(600, 800), (1500, 440)])
 def test_level_items_from_global_memory_bit_exact(gpu, port, rows_bins):
     import gaffa_amd
     from oracle.oracle import TASK_DTYPE
