@@ -65,12 +65,15 @@ scrunch_kernel(const T* __restrict__ data, uint64_t stride, uint64_t factor,
 // samples at f = 2 takes 39 us so, 44 us with 4 full workgroups.
 constexpr uint32_t kScrunchSpan = 4096;
 constexpr uint32_t kScrunchGroups = 1024;
-// Past this factor a wave per output keeps all lanes busy and is the faster one
-// where its waves fill the chip.  Detrending, wave per output against spans, us: 16
-// series of 2^20 samples at f = 104 108, 97; 256 92, 89; 309 91, 94; 700 86, 92; one
-// series at f = 309 (3393 outputs) 43, 44; at 1000 (1048 outputs) 42, 41; at 3000
-// (349) 55, 47.
-constexpr uint32_t kScrunchWave = 256;
+// Past some factor a wave per output keeps all lanes busy and is the faster one
+// where its waves fill the chip: past 256 (whose outputs divide a span), or past 400
+// where the plane is large and the spans' longer bursts count.  Detrending, wave per
+// output against spans, us: 64 series of 131072 samples at f = 256 66, 65; 309 66, 69;
+// 16 of 2^20 at 309 91, 94; 700 86, 92; 64 of 2^20 at 309 305, 302; 512 of 2^22 at 257
+// 10770, 10170; 309 10230, 10040; 400 10070, 9960; 600 9700, 9870; one of 2^20 at 309
+// (3393 outputs) 43, 44; 1000 (1048 outputs) 42, 41; 3000 (349) 55, 47.
+constexpr uint32_t kScrunchWave = 256, kScrunchWaveLarge = 400;
+constexpr uint64_t kScrunchLarge = 1ull << 25;  // samples of all series
 constexpr uint32_t kScrunchWaveOutputs = 2048;
 
 __global__ void __launch_bounds__(kThreads)
@@ -816,7 +819,9 @@ void run(const gaffa_hip_preprocess_args* a, void* workspace, hipStream_t st) {
     if (f > 1) {
       if constexpr (std::is_same_v<T, uint32_t>) {
         const uint64_t all = a->nseries * l.m;
-        if (f <= kScrunchSpan && (f <= kScrunchWave || all < kScrunchWaveOutputs)) {
+        const uint32_t wave =
+            a->nseries * a->nsamples < kScrunchLarge ? kScrunchWave : kScrunchWaveLarge;
+        if (f <= kScrunchSpan && (f <= wave || all < kScrunchWaveOutputs)) {
           const uint32_t outputs = static_cast<uint32_t>(std::min<uint64_t>(
               kScrunchSpan / f, std::max<uint64_t>(1, all / kScrunchGroups)));
           uint32_t lanes = 1;  // about one output per group of lanes

@@ -31,6 +31,9 @@ def test_scrunch_factors(gpu, port, factor):
     (257, 7, 292),      # spans (2044 outputs) ...
     (257, 7, 293),      # ... and a wave per output (2051)
     (1000, 23, 101),
+    (400, 8, 10486),    # spans in a large plane (2^25 samples) ...
+    (401, 8, 10460),    # ... and a wave per output
+    (400, 8, 10485),    # a wave per output in the largest plane below
 ])
 def test_scrunch_outputs(gpu, port, factor, ns, outputs):
     """Both sides of the lines between fewer and more outputs a workgroup and between
