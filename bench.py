@@ -44,38 +44,46 @@ HBM_PEAK_GBS = 8000.0
 
 def kernel_bytes(workload, pipe, ntiles: int, npeaks: int) -> dict:
     """Algorithmic HBM bytes per launch of each hot kernel: the minimum any
-    implementation must move, counted as the search's roofline model does:
+    implementation of it must move, each input read once and each output written
+    once:
 
     dedisperse   one launch for all DM trials: the uint8 filterbank once
                  (nsamples * nchans) + the uint32 plane once (4 * ndm * n_out)
-    ffa_prepare  per series and prepare group: the float series once (4 n) +
-                 the group's prepared copy once (4 P_g)
+    ffa_prepare  per series: the float series once (4 n) + each downsampled
+                 group's prepared copy once (4 P_g)
     ffa_subtree  per series and task of two or more rows: its prepared rows
                  read once (4 rows bins); intermediate levels count zero
-    ffa_levels   intermediate levels only: zero algorithmic bytes (the counter
-                 traffic is reported beside it)
+    ffa_levels   per series, task and global pass: the rows of one depth in and
+                 of another out (8 rows bins), averaged over the launches
     ffa_detect   per series and one-row task: its row once (4 bins) + 24 B per
                  peak record
-    ffa          the whole FFA stage: the sum of the four above
+    ffa          the whole FFA stage: the sum of prepare, subtree and detect;
+                 the levels between count zero, as another algorithm need not
+                 write them
     """
     import numpy as np
+
+    from gaffa_amd import _core
 
     t = pipe.ffa_plan.tasks
     n_out, ndm = pipe.out_nsamples, pipe.ndm
     rb = t["rows"].astype(np.float64) * t["bins"]
     series_per_tile = ndm / ntiles
-    prep = 0.0
+    prep = 4.0 * n_out
     for f in np.unique(t["downsample_factor"]):
-        prep += 4.0 * n_out + 4.0 * float(t["prepared_nsamples"][t["downsample_factor"] == f][0])
+        if f != 1.0:
+            prep += 4.0 * float(t["prepared_nsamples"][t["downsample_factor"] == f][0])
     subtree = 4.0 * float(rb[t["rows"] >= 2].sum())
     detect = 4.0 * float(rb[t["rows"] < 2].sum())
     nlev = max(1, pipe.ffa_layout["level_launches"])
+    items = _core._ffa_level_layout(pipe.ffa_plan)["items"]  # task, depth and levels, first, rows
+    level = 8.0 * float((items[:, 3].astype(np.float64) * t["bins"][items[:, 0]]).sum())
     per_tile_peaks = 24.0 * npeaks / ntiles
     return {
         "dedisperse": (1, workload.nsamples * workload.nchans + 4.0 * ndm * n_out),
         "ffa_prepare": (ntiles, prep * series_per_tile),
         "ffa_subtree": (ntiles, subtree * series_per_tile),
-        "ffa_levels": (ntiles * nlev, 0.0),
+        "ffa_levels": (ntiles * nlev, level * series_per_tile / nlev),
         "ffa_detect": (ntiles, detect * series_per_tile + per_tile_peaks),
         "ffa": (ntiles, (prep + subtree + detect) * series_per_tile + per_tile_peaks),
     }

@@ -1095,8 +1095,9 @@ struct Desc2 {
 //   L = 2: (v0 + v1) + (v2 + v3)
 //   L = 3: ((v0 + v1) + (v2 + v3)) + ((v4 + v5) + (v6 + v7))
 // with v_j = leaf_j[(p + R_j) mod b]; the depth d + 1 .. d + L - 1 values are
-// the FP32 sums in between and are never written.  The host builds each
-// row's leaves (gaffa_hip_ffa_level_row) once per plan.
+// the FP32 sums in between and are never written.  Each row's leaves
+// (gaffa_hip_ffa_level_row) are built once per plan, on the device
+// (ffa_level_rows_kernel).
 __host__ __device__ __forceinline__ gaffa_hip_ffa_level_row level_leaves(uint32_t task_rows,
                                                                          uint32_t depth,
                                                                          uint32_t levels,
@@ -1579,8 +1580,8 @@ int64_t subtree_gain(uint32_t rows, uint32_t bins) {
 
 // Leaf rows of 8 level items a workgroup, a thread per row: stores bound it (36 MB
 // at 2^22 samples).  On the host, with the merge tables that plans in registers
-// never read, they were most of a one-shot search of one such series: 23 ms of
-// host work and upload, 3.6 ms in all with this.
+// never read, they were most of a one-shot search of one such series: 25.2 ms a
+// call, 3.65 with this.
 constexpr uint32_t kTableItems = 8;
 __global__ void __launch_bounds__(kTableItems * kLevelRowsMax)
 ffa_level_rows_kernel(const gaffa_hip_ffa_task* __restrict__ tasks,
