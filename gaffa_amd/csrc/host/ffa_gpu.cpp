@@ -463,6 +463,13 @@ GpuFfaProgram::GpuFfaProgram(const FfaSearchPlan& plan, const GpuFfaProgramOptio
   desc_.work_stride = exec_plan_.work_stride();
 }
 
+GpuFfaProgram::~GpuFfaProgram() {
+  GpuDeviceMemory::release_together(
+      {d_groups_.memory(), d_tasks_.memory(), d_subtree_.memory(), d_level_.memory(),
+       d_terminal_.memory(), d_level_spans_.memory(), d_level_rows_.memory(), d_merges_.memory(),
+       prepared_.memory(), work_.memory(), peaks_.memory(), peak_count_.memory()});
+}
+
 std::size_t GpuFfaProgram::workspace_bytes() const noexcept {
   return prepared_.bytes() + work_.bytes() + peaks_.bytes();
 }

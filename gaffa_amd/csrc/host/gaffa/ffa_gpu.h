@@ -161,6 +161,7 @@ class GpuFfaProgram {
                          const GpuFfaExecutionOptions& execution_options = {});
   GpuFfaProgram(GpuFfaProgram&&) noexcept = default;
   GpuFfaProgram& operator=(GpuFfaProgram&&) noexcept = default;
+  ~GpuFfaProgram();
 
   const GpuFfaExecutionPlan& execution_plan() const noexcept { return exec_plan_; }
   int device_id() const noexcept { return program_.device_id; }

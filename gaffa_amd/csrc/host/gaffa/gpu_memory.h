@@ -7,6 +7,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <initializer_list>
 #include <limits>
 #include <stdexcept>
 #include <string>
@@ -67,13 +68,16 @@ class GpuDeviceMemory {
   ~GpuDeviceMemory();
 
   void reset();
+  // Releases allocations of one device after one wait for it, for objects that own
+  // many (a wait costs about 1 us, 12 of them were 2 % of a search of 8192 samples).
+  static void release_together(std::initializer_list<GpuDeviceMemory*> blocks) noexcept;
   void* data() noexcept { return data_; }
   const void* data() const noexcept { return data_; }
   std::size_t bytes() const noexcept { return bytes_; }
   int device_id() const noexcept { return device_id_; }
 
  private:
-  void release_noexcept() noexcept;
+  bool release_noexcept(bool idle = false) noexcept;  // whether the device is idle after it
   void* data_ = nullptr;
   std::size_t bytes_ = 0;
   std::size_t block_ = 0;  // size of the allocation, >= bytes_
@@ -94,6 +98,7 @@ class GpuDeviceBuffer {
   std::size_t size() const noexcept { return count_; }
   std::size_t bytes() const noexcept { return memory_.bytes(); }
   int device_id() const noexcept { return memory_.device_id(); }
+  GpuDeviceMemory* memory() noexcept { return &memory_; }
 
   GpuSpan<T> as_span() noexcept { return GpuSpan<T>{data(), count_, device_id()}; }
   GpuSpan<const T> as_span() const noexcept {

@@ -50,7 +50,8 @@ class DeviceCache {
     return p;
   }
 
-  int give(int device, void* data, std::size_t bytes) noexcept {
+  // `idle`: the device is known to be done with the block.
+  int give(int device, void* data, std::size_t bytes, bool idle = false) noexcept {
     std::list<Block> own, out;
     Device* held = nullptr;
     try {  // all that can fail for want of host memory comes before the block is listed
@@ -61,7 +62,7 @@ class DeviceCache {
     }
     if (bytes > held->limit) return gaffa_hip_free(data);
     // no kernel of any stream uses the block after this, as with hipFree
-    const int status = wait_for_device();
+    const int status = idle ? GAFFA_HIP_OK : wait_for_device();
     if (status != GAFFA_HIP_OK) {
       (void)gaffa_hip_free(data);
       return status;
@@ -221,16 +222,22 @@ void GpuDeviceMemory::reset() {
   bytes_ = 0;
 }
 
-void GpuDeviceMemory::release_noexcept() noexcept {
-  if (data_ == nullptr) return;
+void GpuDeviceMemory::release_together(std::initializer_list<GpuDeviceMemory*> blocks) noexcept {
+  bool idle = false;
+  for (GpuDeviceMemory* m : blocks) idle = m->release_noexcept(idle);
+}
+
+bool GpuDeviceMemory::release_noexcept(bool idle) noexcept {
+  if (data_ == nullptr) return idle;
   int32_t cur = 0;
   const bool switch_dev = gaffa_hip_get_device(&cur) == 0 && cur != device_id_;
   if (switch_dev) (void)gaffa_hip_set_device(device_id_);
-  (void)DeviceCache::get().give(device_id_, data_, block_);
+  idle = DeviceCache::get().give(device_id_, data_, block_, idle) == GAFFA_HIP_OK;
   if (switch_dev) (void)gaffa_hip_set_device(cur);
   data_ = nullptr;
   bytes_ = 0;
   block_ = 0;
+  return idle;
 }
 
 GpuStream GpuStream::create() {

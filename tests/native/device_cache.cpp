@@ -62,8 +62,10 @@ int gaffa_hip_device_info_get(int32_t, gaffa_hip_device_info* out) {
 }
 gaffa_hip_reclaim_fn reclaim = nullptr;
 int gaffa_hip_set_reclaim(gaffa_hip_reclaim_fn f) { return reclaim = f, 0; }
+int waits = 0;  // one-byte allocations
 int gaffa_hip_malloc(void** p, uint64_t bytes) {
   *p = nullptr;
+  waits += bytes == 1;
   if (used + bytes > kMemory && reclaim != nullptr) (void)reclaim(current);
   if (used + bytes > kMemory) return GAFFA_HIP_RUNTIME;
   for (auto& l : live)
@@ -128,6 +130,19 @@ int main() {
   current = 30;
   { gaffa::GpuDeviceMemory a(kMemory / 64), b(kMemory / 48), c(kMemory / 40); }
   expect(used <= kMemory / 32 && used > 0, "more kept than the bound, or nothing", 0);
+  gaffa::release_device_cache();
+  expect(live_count() == 0, "memory lost", 0);
+  // one wait for several; each is kept or freed
+  {
+    gaffa::GpuDeviceMemory a(5000), b(kMemory / 8), c(7000), d(300);
+    a.reset();
+    waits = 0;
+    gaffa::GpuDeviceMemory::release_together({&a, &b, &c, &d});
+    expect(waits == 0 && b.data() == nullptr && d.data() == nullptr, "wait after a free", 0);
+    gaffa::GpuDeviceMemory e(5000), f(7000), g(300);
+    gaffa::GpuDeviceMemory::release_together({&e, &f, &g});
+    expect(waits == 1, "not one wait", waits);
+  }
   gaffa::release_device_cache();
   expect(live_count() == 0, "memory lost", 0);
   // an allocation that needs what is kept gets it
